@@ -93,5 +93,22 @@ __device__ __forceinline__ half_t mx_f16_sat(float v) {
   return (half_t)v;
 }
 
+// 16 int8 -> 16 fp16, exact: byte u = q + 128 placed under exponent 0x64 reads as
+// 1024 + u in fp16; subtracting 1152 leaves q.
+__device__ __forceinline__ void mx_i8_to_f16(int4_t v, half8_t& lo, half8_t& hi) {
+  const half2_t bias = {(half_t)1152.0f, (half_t)1152.0f};
+  half2_t h[8];
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    const uint32_t u = (uint32_t)v[d] ^ 0x80808080u;
+    const uint32_t p0 = __builtin_amdgcn_perm(0x64646464u, u, 0x04010400u);
+    const uint32_t p1 = __builtin_amdgcn_perm(0x64646464u, u, 0x04030402u);
+    h[2 * d] = __builtin_bit_cast(half2_t, p0) - bias;
+    h[2 * d + 1] = __builtin_bit_cast(half2_t, p1) - bias;
+  }
+  lo = (half8_t){h[0][0], h[0][1], h[1][0], h[1][1], h[2][0], h[2][1], h[3][0], h[3][1]};
+  hi = (half8_t){h[4][0], h[4][1], h[5][0], h[5][1], h[6][0], h[6][1], h[7][0], h[7][1]};
+}
+
 static inline int mx_ceil_div(int a, int b) { return (a + b - 1) / b; }
 static inline size_t mx_align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }

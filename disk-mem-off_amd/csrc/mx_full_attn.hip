@@ -63,6 +63,7 @@ struct Carve {
 struct FaWork {
   MxFullAttnViews v;
   MxDenseWork dw;  // projections: entry 0 q, 1 k, 2 v, 3 o
+  float* o_part = nullptr;  // o projection of short inputs: reduction slices 1 ..
   half_t* k16;     // fp16 path: keys [n_kv][Tp][DP] (Tp = T padded to 32 keys, DP = hd padded to 32)
   half_t* v16t;    // fp16 path: values per 32-key tile, transposed [n_kv][Tp / 32][DP][32]
 };
@@ -90,6 +91,7 @@ int layout(const MxFullAttnDesc* d, int T, void* ws, FaWork* w, size_t* total) {
   t.v.y = (float*)c.take(Tn * m.H * 4);
   char* dwb = (char*)c.take(mx_dense_work_bytes((int)Tn, d->weight_dtype, 4));
   mx_dense_work_carve(dwb, (int)Tn, d->weight_dtype, 4, &t.dw);
+  t.o_part = (float*)c.take(mx_proj_part_bytes(d->weight_dtype, (int)Tn, m.H, m.od));
   if (!f32) {
     const size_t tp = (Tn + FA_TPAD - 1) / FA_TPAD * FA_TPAD, dp = (size_t)(m.hd + 31) / 32 * 32;
     t.k16 = (half_t*)c.take((size_t)m.nkv * tp * dp * 2);
@@ -1002,14 +1004,9 @@ int attn_launch(const float* qg, const float* kk, const float* vv, const FaDims&
   return MX_ERR_UNSUPPORTED;
 }
 
-__global__ __launch_bounds__(256) void k_fa_residual(const float* __restrict__ x,
-                                                     const float* __restrict__ y, long n4,
-                                                     float* __restrict__ out) {
-  const long i = (long)blockIdx.x * 256 + threadIdx.x;
-  if (i < n4) {
-    const float4 a = ((const float4*)x)[i], b = ((const float4*)y)[i];
-    ((float4*)out)[i] = make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
-  }
+// Whether the projection with reduction length K needs the grouped kernels' tables.
+bool on_grouped(int wdt, int T, int K) {
+  return !mx_proj_ok(wdt, T, K) && !mx_dense_on_gemm(wdt, T, K);
 }
 
 int check_weights(const MxFullAttnDesc* d, const MxFullAttnWeights* w) {
@@ -1029,21 +1026,28 @@ int run_stage(int st, const MxFullAttnDesc* d, const MxFullAttnWeights* w, const
   const bool f32 = wdt == MX_DT_F32;
   const void* h = f32 ? (const void*)k.v.h32 : k.v.h16;
   switch (st) {
-    case 0: {
-      MxDenseEntries e = {};
-      e.e[0].down = w->q_w;
-      e.e[0].down_scale = w->q_scale;
-      e.e[1].down = w->k_w;
-      e.e[1].down_scale = w->k_scale;
-      e.e[2].down = w->v_w;
-      e.e[2].down_scale = w->v_scale;
-      e.e[3].down = w->o_w;
-      e.e[3].down_scale = w->o_scale;
-      MX_TRY(mx_dense_setup(k.dw, e, T, s));
+    case 0:
+      if (on_grouped(wdt, T, m.H) || on_grouped(wdt, T, m.od)) {
+        MxDenseEntries e = {};
+        e.e[0].down = w->q_w;
+        e.e[0].down_scale = w->q_scale;
+        e.e[1].down = w->k_w;
+        e.e[1].down_scale = w->k_scale;
+        e.e[2].down = w->v_w;
+        e.e[2].down_scale = w->v_scale;
+        e.e[3].down = w->o_w;
+        e.e[3].down_scale = w->o_scale;
+        MX_TRY(mx_dense_setup(k.dw, e, T, s));
+      }
       return mx_rmsnorm_launch(x, w->norm_w, d->param_dtype, d->eps, T, m.H, k.v.h32, k.v.h16,
                                s);
-    }
     case 1:
+      if (mx_proj_ok(wdt, T, m.H)) {  // q, k and v share h: one launch
+        const MxProjSeg g[3] = {{w->q_w, w->q_scale, k.v.qg, m.qw, m.qw},
+                                {w->k_w, w->k_scale, k.v.k, m.kw, m.kw},
+                                {w->v_w, w->v_scale, k.v.v, m.kw, m.kw}};
+        return mx_proj(wdt, h, T, m.H, g, 3, 1, nullptr, s);
+      }
       if (mx_dense_on_gemm(wdt, T, m.H)) {  // q, k and v share h: one GEMM launch
         const MxGemmSeg g[3] = {{w->q_w, k.v.qg, m.qw, m.qw},
                                 {w->k_w, k.v.k, m.kw, m.kw},
@@ -1052,10 +1056,10 @@ int run_stage(int st, const MxFullAttnDesc* d, const MxFullAttnWeights* w, const
       }
       return mx_project(k.dw, 0, wdt, w->q_w, T, m.qw, m.H, h, k.v.qg, s);
     case 2:
-      if (mx_dense_on_gemm(wdt, T, m.H)) return MX_OK;  // with q in stage 1
+      if (!on_grouped(wdt, T, m.H)) return MX_OK;  // with q in stage 1
       return mx_project(k.dw, 1, wdt, w->k_w, T, m.kw, m.H, h, k.v.k, s);
     case 3:
-      if (mx_dense_on_gemm(wdt, T, m.H)) return MX_OK;
+      if (!on_grouped(wdt, T, m.H)) return MX_OK;
       return mx_project(k.dw, 2, wdt, w->v_w, T, m.kw, m.H, h, k.v.v, s);
     case 4: {
       // Long inputs: one block per token (4096 tokens: 34 us against 41 us with 4 rows per
@@ -1077,20 +1081,21 @@ int run_stage(int st, const MxFullAttnDesc* d, const MxFullAttnWeights* w, const
     case 5:
       return attn_launch(k.v.qg, k.v.k, k.v.v, m, T, k.v.act, !f32, k.k16, k.v16t, s);
     case 6:
+      if (mx_proj_ok(wdt, T, m.od)) {
+        const MxProjSeg g{w->o_w, w->o_scale, k.v.y, m.H, m.H};
+        return mx_proj(wdt, k.v.act, T, m.od, &g, 1, mx_proj_slices(wdt, m.H, m.od), k.o_part, s);
+      }
       if (mx_dense_on_gemm(wdt, T, m.od)) {  // out = x + act W_o^T in the GEMM epilogue
         if (!x || !out) return MX_ERR_INVALID;
         const MxGemmSeg g{w->o_w, out, m.H, m.H, nullptr, x};
         return mx_gemm_f16(k.v.act, T, m.od, &g, 1, s);
       }
       return mx_project(k.dw, 3, wdt, w->o_w, T, m.H, m.od, k.v.act, k.v.y, s);
-    case 7: {
+    case 7:
       if (mx_dense_on_gemm(wdt, T, m.od)) return MX_OK;  // added in stage 6
-      const long n4 = (long)T * m.H / 4;
-      mx_clear_error();
-      hipLaunchKernelGGL(k_fa_residual, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, x,
-                         k.v.y, n4, out);
-      return mx_launch_status();
-    }
+      return mx_residual(x, k.v.y, k.o_part,
+                         mx_proj_ok(wdt, T, m.od) ? mx_proj_slices(wdt, m.H, m.od) : 1,
+                         (long)T * m.H, out, s);
     default:
       return MX_ERR_INVALID;
   }

@@ -153,6 +153,30 @@ int mx_gemm_f32_slices(const float* a, int M, int K, const MxGemmSeg* segs, int 
 int mx_gemm_f16x2_slices(const void* a_hi, const void* a_lo, int M, int K, const MxGemmSeg* segs,
                          int nseg, int kslice, long yslice, hipStream_t s);
 
+// Projections of short inputs (mx_proj.hip): fp16 or per-row int8 weights, up to
+// MX_PROJ_MAX_TOKENS tokens.  With `slices` > 1 (one segment only) the reduction is split
+// over grid slices: slice 0 goes to the segment's y, slice i to part + (i - 1) T n; the
+// residual sum adds them.
+#define MX_PROJ_MAX_TOKENS 64
+#define MX_PROJ_MAX_SLICES 4
+struct MxProjSeg {
+  const void* w;      // [n, K] row-major, 16-byte aligned
+  const void* scale;  // fp16 [n] for MX_DT_I8
+  float* y;           // [T, ldy]
+  int n;
+  int ldy;
+};
+bool mx_proj_ok(int wdt, int T, int K);
+int mx_proj_slices(int wdt, int N, int K);
+// Bytes of `part` for T tokens (does not shrink as T grows).
+size_t mx_proj_part_bytes(int wdt, int T, int N, int K);
+int mx_proj(int wdt, const void* a, int T, int K, const MxProjSeg* segs, int nseg, int slices,
+            float* part, hipStream_t s);
+// out = x + y (+ the slices in `part`; y then holds the sum) over n floats, n % 4 == 0, all
+// 16-byte aligned; out may alias x.
+int mx_residual(const float* x, float* y, const float* part, int slices, long n, float* out,
+                hipStream_t s);
+
 // Workspace pieces of the dense projections of an attention block (device pointers):
 // expert-table entries (one per projection), single-group m-tile tables and ones[T] for
 // the grouped-GEMM kernels.  Long inputs with fp16 weights run on mx_gemm_f16 instead.

@@ -67,6 +67,7 @@ struct Carve {
 struct LaWork {
   MxLinearAttnViews v;
   MxDenseWork dw;      // projections: entry 0 qkvz, 1 ba, 2 out
+  float* out_part = nullptr;  // out projection of short inputs: reduction slices 1 ..
   void* chunk_ws = nullptr;  // chunked scan: coefficients and chunk states (NULL: sequential)
 };
 
@@ -91,6 +92,7 @@ int layout(const MxLinearAttnDesc* d, int T, void* ws, LaWork* w, size_t* total)
   t.v.y = (float*)c.take(Tn * m.H * 4);
   char* dwb = (char*)c.take(mx_dense_work_bytes((int)Tn, d->weight_dtype, 3));
   mx_dense_work_carve(dwb, (int)Tn, d->weight_dtype, 3, &t.dw);
+  t.out_part = (float*)c.take(mx_proj_part_bytes(d->weight_dtype, (int)Tn, m.H, m.vd));
   const size_t cb = mx_la_chunk_ws_bytes((int)Tn, m.n, m.dk, m.dv);
   t.chunk_ws = cb ? c.take(cb) : nullptr;
   if (w) *w = t;
@@ -624,14 +626,9 @@ __global__ __launch_bounds__(256) void k_la_gated_norm(const float* __restrict__
   }
 }
 
-__global__ __launch_bounds__(256) void k_la_residual(const float* __restrict__ x,
-                                                     const float* __restrict__ y, long n4,
-                                                     float* __restrict__ out) {
-  const long i = (long)blockIdx.x * 256 + threadIdx.x;
-  if (i < n4) {
-    const float4 a = ((const float4*)x)[i], b = ((const float4*)y)[i];
-    ((float4*)out)[i] = make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
-  }
+// Whether the projection with reduction length K needs the grouped kernels' tables.
+bool on_grouped(int wdt, int T, int K) {
+  return !mx_proj_ok(wdt, T, K) && !mx_dense_on_gemm(wdt, T, K);
 }
 
 int check_weights(const MxLinearAttnDesc* d, const MxLinearAttnWeights* w) {
@@ -652,26 +649,32 @@ int run_stage(int st, const MxLinearAttnDesc* d, const MxLinearAttnWeights* w, c
   const bool f32 = wdt == MX_DT_F32;
   const void* h = f32 ? (const void*)k.v.h32 : k.v.h16;
   switch (st) {
-    case 0: {
-      MxDenseEntries e = {};
-      e.e[0].down = w->qkvz_w;
-      e.e[0].down_scale = w->qkvz_scale;
-      e.e[1].down = w->ba_w;
-      e.e[1].down_scale = w->ba_scale;
-      e.e[2].down = w->out_w;
-      e.e[2].down_scale = w->out_scale;
-      MX_TRY(mx_dense_setup(k.dw, e, T, s));
+    case 0:
+      if (on_grouped(wdt, T, m.H) || on_grouped(wdt, T, m.vd)) {
+        MxDenseEntries e = {};
+        e.e[0].down = w->qkvz_w;
+        e.e[0].down_scale = w->qkvz_scale;
+        e.e[1].down = w->ba_w;
+        e.e[1].down_scale = w->ba_scale;
+        e.e[2].down = w->out_w;
+        e.e[2].down_scale = w->out_scale;
+        MX_TRY(mx_dense_setup(k.dw, e, T, s));
+      }
       return mx_rmsnorm_launch(x, w->norm_w, d->param_dtype, d->eps, T, m.H, k.v.h32, k.v.h16,
                                s);
-    }
     case 1:
+      if (mx_proj_ok(wdt, T, m.H)) {  // qkvz and ba share h: one launch
+        const MxProjSeg g[2] = {{w->qkvz_w, w->qkvz_scale, k.v.qkvz, m.W1, m.W1},
+                                {w->ba_w, w->ba_scale, k.v.ba, m.W2, m.W2}};
+        return mx_proj(wdt, h, T, m.H, g, 2, 1, nullptr, s);
+      }
       if (mx_dense_on_gemm(wdt, T, m.H)) {  // qkvz and ba share h: one GEMM launch
         const MxGemmSeg g[2] = {{w->qkvz_w, k.v.qkvz, m.W1, m.W1}, {w->ba_w, k.v.ba, m.W2, m.W2}};
         return mx_gemm_f16(h, T, m.H, g, 2, s);
       }
       return mx_project(k.dw, 0, wdt, w->qkvz_w, T, m.W1, m.H, h, k.v.qkvz, s);
     case 2:
-      if (mx_dense_on_gemm(wdt, T, m.H)) return MX_OK;  // with qkvz in stage 1
+      if (!on_grouped(wdt, T, m.H)) return MX_OK;  // with qkvz in stage 1
       return mx_project(k.dw, 1, wdt, w->ba_w, T, m.W2, m.H, h, k.v.ba, s);
     case 3: {
       const dim3 grid(mx_ceil_div(m.C + m.n, 256), mx_ceil_div(T, LA_TT));
@@ -705,20 +708,22 @@ int run_stage(int st, const MxLinearAttnDesc* d, const MxLinearAttnWeights* w, c
                            f32 ? nullptr : (half_t*)k.v.act);
       return mx_launch_status();
     case 6:
+      if (mx_proj_ok(wdt, T, m.vd)) {
+        const MxProjSeg g{w->out_w, w->out_scale, k.v.y, m.H, m.H};
+        return mx_proj(wdt, k.v.act, T, m.vd, &g, 1, mx_proj_slices(wdt, m.H, m.vd), k.out_part,
+                       s);
+      }
       if (mx_dense_on_gemm(wdt, T, m.vd)) {  // out = x + act W_out^T in the GEMM epilogue
         if (!x || !out) return MX_ERR_INVALID;
         const MxGemmSeg g{w->out_w, out, m.H, m.H, nullptr, x};
         return mx_gemm_f16(k.v.act, T, m.vd, &g, 1, s);
       }
       return mx_project(k.dw, 2, wdt, w->out_w, T, m.H, m.vd, k.v.act, k.v.y, s);
-    case 7: {
+    case 7:
       if (mx_dense_on_gemm(wdt, T, m.vd)) return MX_OK;  // added in stage 6
-      const long n4 = (long)T * m.H / 4;
-      mx_clear_error();
-      hipLaunchKernelGGL(k_la_residual, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, x,
-                         k.v.y, n4, out);
-      return mx_launch_status();
-    }
+      return mx_residual(x, k.v.y, k.out_part,
+                         mx_proj_ok(wdt, T, m.vd) ? mx_proj_slices(wdt, m.H, m.vd) : 1,
+                         (long)T * m.H, out, s);
     default:
       return MX_ERR_INVALID;
   }

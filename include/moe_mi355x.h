@@ -368,7 +368,8 @@ typedef struct MxLinearAttnViews {
  * projections run on the dense MFMA GEMM: ba is computed in the qkvz launch (stage 2 is
  * then empty, and the _profiled events report ba's time under qkvz), and out = x +
  * act W_out^T is formed in the out launch's epilogue (stage 7 is empty and the view y is
- * not written).                                                                        */
+ * not written).  With fp16 or int8 weights and T <= 64 ba is computed in the qkvz launch
+ * too.                                                                                 */
 #define MX_LA_N_STAGES 8
 
 int mx_linear_attn_workspace_size(const MxLinearAttnDesc* desc, int32_t tokens,
@@ -438,7 +439,8 @@ typedef struct MxFullAttnViews {
  * projections run on the dense MFMA GEMM: k and v are computed in the q launch (stages 2
  * and 3 are then empty, and the _profiled events report their time under q), and out =
  * x + act W_o^T is formed in the o launch's epilogue (stage 7 is empty and the view y is
- * not written).                                                                        */
+ * not written).  With fp16 or int8 weights and T <= 64 k and v are computed in the q
+ * launch too.                                                                          */
 #define MX_FA_N_STAGES 8
 
 int mx_full_attn_workspace_size(const MxFullAttnDesc* desc, int32_t tokens, size_t* nbytes);

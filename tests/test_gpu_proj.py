@@ -1,0 +1,120 @@
+"""Projections of short inputs (``mx_proj.hip``) inside the attention blocks, against float64
+products of the device's own fp16 activations.
+
+Sizes where the kernel can go wrong: token counts at the edges of its 16-row tiles, row
+counts that are no multiple of its 16- and 32-column tiles (one of them leading to rows that
+are not 16-byte aligned), reduction lengths with a partial last chunk, and a reduction long
+enough to be split over grid slices.  Bound: the products of fp16 (int8) pairs are exact in
+fp32, so only the fp32 sums round: at most (K + 16) 2^-24 of the sum of magnitudes, plus the
+row scale's multiplication for int8."""
+import numpy as np
+import pytest
+
+from moe_mi355x import synthetic as syn
+from moe_mi355x.full_attn import DeviceFullAttnLayer
+from moe_mi355x.linear_attn import DeviceLinearAttnLayer
+from moe_mi355x.moe import read_device
+from moe_mi355x.quantize import quantize_rows_int8
+from oracle import full_attn_oracle as fa
+from oracle import linear_attn_oracle as la
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def mi355x():
+    from moe_mi355x.backends import MI355XBackend
+
+    return MI355XBackend(0)
+
+
+@pytest.fixture(scope="module")
+def stream(mi355x):
+    s = mi355x.create_stream("test-proj")
+    yield s
+    mi355x.destroy_stream(s)
+
+
+def _weights(t, names, wdt):
+    """Quantises ``names`` in place for int8; returns name -> (values, row scale), float64."""
+    out = {}
+    for n in names:
+        if wdt == "int8":
+            t[n], t[n + "_scale"] = quantize_rows_int8(t[n].astype(np.float32))
+            out[n] = (t[n].astype(np.float64), t[n + "_scale"].astype(np.float64)[:, None])
+        else:
+            out[n] = (t[n].astype(np.float64), 1.0)
+    return out
+
+
+def _check(name, got, a, weight):
+    w, scale = weight
+    k = a.shape[1]
+    want = a @ (w * scale).T
+    bound = ((k + 16) * 2.0 ** -24 + 2.0 ** -23) * (np.abs(a) @ (np.abs(w) * scale).T) + 1e-30
+    worst = float(np.max(np.abs(got - want) / bound))
+    print(f"    {name} K={k}: worst error {worst:.3f} of the bound", flush=True)
+    assert worst <= 1.0, name
+
+
+@pytest.mark.parametrize("wdt", ["float16", "int8"])
+@pytest.mark.parametrize("T", [1, 15, 16, 17, 32, 33, 64])
+def test_linear_attention_projections(mi355x, stream, wdt, T):
+    # qkvz 3 * 2 * (32 + 512) = 3264 rows of 208, ba 99 rows, out 208 rows of 1536 (sliced)
+    shape = syn.LinearAttnShape(208, 3, 32, 512, 4, 1e-6)
+    print(f"[gpu] linear attention projections {wdt} T={T}", flush=True)
+    t = syn.make_linear_attn_tensors(shape, 90 + T, weight_dtype=np.float16, norm_noise=0.1)
+    w = _weights(t, (la.QKVZ, la.BA, la.OUT), wdt)
+    x = syn.make_inputs(91 + T, T, shape.hidden)
+    layer = DeviceLinearAttnLayer.from_host(mi355x, t, stream)
+    try:
+        out = layer.forward_numpy(x, shape.eps)
+        v = layer.runner.views(layer.desc(shape.eps), T)
+
+        def read(p, dt, n):
+            return read_device(mi355x, p, dt, T * n, stream).reshape(T, n).astype(np.float64)
+
+        vd = shape.n_heads * shape.head_dim_v
+        h, act = read(v.h16, np.float16, shape.hidden), read(v.act, np.float16, vd)
+        qkvz, ba = read(v.qkvz, np.float32, shape.qkvz_rows), read(v.ba, np.float32, shape.ba_rows)
+        y = read(v.y, np.float32, shape.hidden)
+    finally:
+        layer.close()
+    _check("qkvz", qkvz, h, w[la.QKVZ])
+    _check("ba", ba, h, w[la.BA])
+    _check("out", y, act, w[la.OUT])
+    assert np.array_equal(out, x + y.astype(np.float32))
+
+
+@pytest.mark.parametrize("wdt", ["float16", "int8"])
+@pytest.mark.parametrize("T", [1, 16, 31, 48, 64])
+def test_full_attention_projections(mi355x, stream, wdt, T):
+    # q 2 * 6 * 20 = 240 rows of 272, k and v 40 rows, o 272 rows of 120 / int8 6 * 24 = 144
+    hd = 20 if wdt == "float16" else 24
+    s = syn.FullAttnShape(272, 6, 2, hd, 0.5, 10000.0, 1e-6)
+    print(f"[gpu] full attention projections {wdt} T={T}", flush=True)
+    t = syn.make_full_attn_tensors(s, 70 + T, weight_dtype=np.float16, norm_noise=0.1)
+    w = _weights(t, (fa.Q, fa.K, fa.V, fa.O), wdt)
+    x = syn.make_inputs(71 + T, T, s.hidden)
+    layer = DeviceFullAttnLayer.from_host(mi355x, t, s.n_heads, s.n_kv_heads, s.head_dim,
+                                          s.rotary_dim, s.rope_theta, stream)
+    try:
+        out = layer.forward_numpy(x, s.eps)
+        v = layer.runner.views(layer.desc(s.eps), T)
+
+        def read(p, dt, n):
+            return read_device(mi355x, p, dt, T * n, stream).reshape(T, n).astype(np.float64)
+
+        od, kw = s.n_heads * s.head_dim, s.n_kv_heads * s.head_dim
+        h, act = read(v.h16, np.float16, s.hidden), read(v.act, np.float16, od)
+        gate = read(v.qg, np.float32, 2 * od)[:, od:]
+        vv, y = read(v.v, np.float32, kw), read(v.y, np.float32, s.hidden)
+    finally:
+        layer.close()
+    # q and k are normalised and rotated in place after the projection; the gate half of the
+    # q projection and v are left as they were
+    wq, sq = w[fa.Q]
+    _check("gate", gate, h, (wq[od:], sq[od:] if wdt == "int8" else sq))
+    _check("v", vv, h, w[fa.V])
+    _check("o", y, act, w[fa.O])
+    assert np.array_equal(out, x + y.astype(np.float32))
