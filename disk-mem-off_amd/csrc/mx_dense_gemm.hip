@@ -390,7 +390,50 @@ int prepare(GemmArgs& args, const void* a, int M, int K, int es, const MxGemmSeg
   return MX_OK;
 }
 
+// fp16 products on 128 x 128 tiles.  A stage of one block is paced by the latency of its
+// copies (0.6 us with 48 blocks on the whole chip as with 256), so the tiles are kept in
+// flight as the block count allows: up to one block per CU four stage slots and 8 waves
+// (Qwen3-Next, 4096 tokens, k and v: 29.6 us with 4 waves, 28.6 with 8; 300 tokens, q + k +
+// v: 27.4 and 26.9); with more blocks than CUs two blocks per CU with two slots each (q + k +
+// v of 777 tokens, 504 blocks: 54 -> 41 us, of 1500 tokens 99 -> 74; qkvz + ba of 300 tokens
+// 54 -> 44.6, of 1000 tokens 157 -> 122 us, against rounds of one block per CU).
+int launch_small(GemmArgs& args, const MxGemmSeg* segs, int nseg, int splits, hipStream_t s) {
+  long blocks = 0;
+  for (int i = 0; i < nseg; ++i)
+    blocks += (long)mx_ceil_div(args.M, 128) * mx_ceil_div(segs[i].n, 128);
+  if (blocks * splits > 256)
+    return launch<half_t, false, 128, 128, 64, 64, 2, 2>(args, segs, nseg, splits, s);
+  return launch<half_t, false, 128, 128, 64, 32, 4, 1>(args, segs, nseg, splits, s);
+}
+
 }  // namespace
+
+// Products of few tiles (the output projections of mid-length inputs) cut their reduction so
+// that the tiles times the slices fill the CUs once: 2048 columns over 4096, 100 tokens 43.5
+// -> 10 us with 8 slices, 300 tokens 44.5 -> 15 with 5, 777 tokens 48 -> 27.8 with 2 (and
+// 4-7 us for the launch that adds the slices and x).  Two blocks per CU (512) gained nothing
+// below 1500 tokens (300: 17.0 + 8.4 us; 777: 25.9 + 9.1).  A slice keeps at least 8 stages.
+int mx_gemm_f16_slice_count(int M, int N, int K) {
+  const int blocks = mx_ceil_div(M, 128) * mx_ceil_div(N, 128);
+  const int nst = K / MX_GEMM_KMULT_F16;
+  int s = MX_GEMM_SLICE_BLOCKS / blocks;
+  if (s > MX_GEMM_MAX_SLICES) s = MX_GEMM_MAX_SLICES;
+  while (s > 1 && nst / s < 8) --s;
+  return s < 1 ? 1 : s;
+}
+
+int mx_gemm_f16_slices(const void* a, int M, int K, const MxGemmSeg* seg, int slices,
+                       hipStream_t s) {
+  if (!seg || slices < 1 || slices > MX_GEMM_MAX_SLICES || seg->ldy != seg->n || seg->res)
+    return MX_ERR_INVALID;
+  const int nst = K / MX_GEMM_KMULT_F16;
+  // Slices of equal length but the last, every one with at least one stage.
+  const int per = mx_ceil_div(nst, slices);
+  if (nst < 1 || (slices - 1) * per >= nst) return MX_ERR_INVALID;
+  GemmArgs args;
+  MX_TRY(prepare(args, a, M, K, 2, seg, 1, per * MX_GEMM_KMULT_F16, (long)M * seg->n));
+  return launch_small(args, seg, 1, slices, s);
+}
 
 #ifndef MX_GEMM_MID
 #define MX_GEMM_MID 1  // 256 x 128 tiles for products that fill whole rounds with them
@@ -405,9 +448,7 @@ int mx_gemm_f16(const void* a, int M, int K, const MxGemmSeg* segs, int nseg, hi
   long cols = 0;
   for (int i = 0; i < nseg; ++i) cols += segs[i].n;
   // 256 x 256 tiles while they give at least two rounds of blocks on 256 CUs; 128 x 128
-  // (four waves, one block per CU with four 32 KiB stage slots: 34 -> 30 us for the k and v
-  // projections of the Qwen3-Next 4096-token attention block against two blocks per CU
-  // with two slots each) otherwise.
+  // otherwise.
   const long big = (long)mx_ceil_div(M, 256) * mx_ceil_div((int)cols, 256);
   if (big < 512) {
     // 256 x 128 tiles (8 waves of 64 x 64, one block per CU) when they fill whole rounds
@@ -415,7 +456,7 @@ int mx_gemm_f16(const void* a, int M, int K, const MxGemmSeg* segs, int nseg, hi
     for (int i = 0; i < nseg; ++i) mid += (long)mx_ceil_div(M, 256) * mx_ceil_div(segs[i].n, 128);
     if (MX_GEMM_MID && mid >= 256 && mid % 256 == 0)
       return launch<half_t, false, 256, 128, 64, 64, 3, 1>(args, segs, nseg, 1, s);
-    return launch<half_t, false, 128, 128, 64, 64, 4, 1>(args, segs, nseg, 1, s);
+    return launch_small(args, segs, nseg, 1, s);
   }
   if (MX_GEMM_TAIL && big % 256) {
     // One 256 x 256 block per CU: the blocks past the last whole round would run as a
@@ -449,7 +490,7 @@ int mx_gemm_f16(const void* a, int M, int K, const MxGemmSeg* segs, int nseg, hi
       MX_TRY(prepare(ah, a, M, K, 2, head, nh, K, 0));
       MX_TRY(prepare(at, a, M, K, 2, tail, nt, K, 0));
       MX_TRY((launch<half_t, false, 256, 256, 128, 64, 2, 1>(ah, head, nh, 1, s)));
-      return launch<half_t, false, 128, 128, 64, 64, 4, 1>(at, tail, nt, 1, s);
+      return launch_small(at, tail, nt, 1, s);
     }
   }
   return launch<half_t, false, 256, 256, 128, 64, 2, 1>(args, segs, nseg, 1, s);

@@ -63,7 +63,6 @@ struct Carve {
 struct FaWork {
   MxFullAttnViews v;
   MxDenseWork dw;  // projections: entry 0 q, 1 k, 2 v, 3 o
-  float* o_part = nullptr;  // o projection of short inputs: reduction slices 1 ..
   half_t* k16;     // fp16 path: keys [n_kv][Tp][DP] (Tp = T padded to 32 keys, DP = hd padded to 32)
   half_t* v16t;    // fp16 path: values per 32-key tile, transposed [n_kv][Tp / 32][DP][32]
 };
@@ -88,10 +87,9 @@ int layout(const MxFullAttnDesc* d, int T, void* ws, FaWork* w, size_t* total) {
   t.v.k = (float*)c.take(Tn * m.kw * 4);
   t.v.v = (float*)c.take(Tn * m.kw * 4);
   t.v.act = c.take(Tn * m.od * (f32 ? 4 : 2));
-  t.v.y = (float*)c.take(Tn * m.H * 4);
+  t.v.y = (float*)c.take(mx_out_rows((int)Tn, m.H) * m.H * 4);
   char* dwb = (char*)c.take(mx_dense_work_bytes((int)Tn, d->weight_dtype, 4));
   mx_dense_work_carve(dwb, (int)Tn, d->weight_dtype, 4, &t.dw);
-  t.o_part = (float*)c.take(mx_proj_part_bytes(d->weight_dtype, (int)Tn, m.H, m.od));
   if (!f32) {
     const size_t tp = (Tn + FA_TPAD - 1) / FA_TPAD * FA_TPAD, dp = (size_t)(m.hd + 31) / 32 * 32;
     t.k16 = (half_t*)c.take((size_t)m.nkv * tp * dp * 2);
@@ -1046,7 +1044,7 @@ int run_stage(int st, const MxFullAttnDesc* d, const MxFullAttnWeights* w, const
         const MxProjSeg g[3] = {{w->q_w, w->q_scale, k.v.qg, m.qw, m.qw},
                                 {w->k_w, w->k_scale, k.v.k, m.kw, m.kw},
                                 {w->v_w, w->v_scale, k.v.v, m.kw, m.kw}};
-        return mx_proj(wdt, h, T, m.H, g, 3, 1, nullptr, s);
+        return mx_proj(wdt, h, T, m.H, g, 3, 1, s);
       }
       if (mx_dense_on_gemm(wdt, T, m.H)) {  // q, k and v share h: one GEMM launch
         const MxGemmSeg g[3] = {{w->q_w, k.v.qg, m.qw, m.qw},
@@ -1081,21 +1079,10 @@ int run_stage(int st, const MxFullAttnDesc* d, const MxFullAttnWeights* w, const
     case 5:
       return attn_launch(k.v.qg, k.v.k, k.v.v, m, T, k.v.act, !f32, k.k16, k.v16t, s);
     case 6:
-      if (mx_proj_ok(wdt, T, m.od)) {
-        const MxProjSeg g{w->o_w, w->o_scale, k.v.y, m.H, m.H};
-        return mx_proj(wdt, k.v.act, T, m.od, &g, 1, mx_proj_slices(wdt, m.H, m.od), k.o_part, s);
-      }
-      if (mx_dense_on_gemm(wdt, T, m.od)) {  // out = x + act W_o^T in the GEMM epilogue
-        if (!x || !out) return MX_ERR_INVALID;
-        const MxGemmSeg g{w->o_w, out, m.H, m.H, nullptr, x};
-        return mx_gemm_f16(k.v.act, T, m.od, &g, 1, s);
-      }
-      return mx_project(k.dw, 3, wdt, w->o_w, T, m.H, m.od, k.v.act, k.v.y, s);
+      return mx_out_project(k.dw, 3, wdt, w->o_w, w->o_scale, T, m.H, m.od, k.v.act, k.v.y, x,
+                            out, s);
     case 7:
-      if (mx_dense_on_gemm(wdt, T, m.od)) return MX_OK;  // added in stage 6
-      return mx_residual(x, k.v.y, k.o_part,
-                         mx_proj_ok(wdt, T, m.od) ? mx_proj_slices(wdt, m.H, m.od) : 1,
-                         (long)T * m.H, out, s);
+      return mx_out_residual(wdt, T, m.H, m.od, k.v.y, x, out, s);
     default:
       return MX_ERR_INVALID;
   }

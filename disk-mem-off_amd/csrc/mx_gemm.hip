@@ -28,7 +28,84 @@ __global__ __launch_bounds__(256) void k_dense_setup(int T, int m_blk, int n_mt,
   if (i < T) ones[i] = 1.f;
 }
 
+// out = x + y, or + the slices of y (n floats each) in slice order; y then receives their sum
+// where it is wanted.
+template <bool SLICED>
+__global__ __launch_bounds__(256) void k_residual(const float* x, float* y, long n4, int slices,
+                                                  bool keep, float* out) {
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n4) return;
+  const float4_t a = ((const float4_t*)x)[i];
+  float4_t b = ((const float4_t*)y)[i];
+  if constexpr (SLICED) {
+    float4_t e[MX_GEMM_MAX_SLICES - 1];
+#pragma unroll
+    for (int s = 1; s < MX_GEMM_MAX_SLICES; ++s)
+      if (s < slices) e[s - 1] = ((const float4_t*)y)[i + s * n4];
+#pragma unroll
+    for (int s = 1; s < MX_GEMM_MAX_SLICES; ++s)
+      if (s < slices) b += e[s - 1];
+    if (keep) ((float4_t*)y)[i] = b;
+  }
+  ((float4_t*)out)[i] = a + b;
+}
+
+static_assert(MX_PROJ_MAX_SLICES <= MX_GEMM_MAX_SLICES, "k_residual adds either's slices");
+
+// Reduction slices of an output projection.
+int out_slices(int wdt, int T, int N, int K) {
+  if (mx_proj_ok(wdt, T, K)) return mx_proj_slices(wdt, N, K);
+  if (mx_dense_on_gemm(wdt, T, K)) return mx_gemm_f16_slice_count(T, N, K);
+  return 1;
+}
+
 }  // namespace
+
+size_t mx_out_rows(int T, int N) {
+  // At least slices x T for every path's slice count, and never less for fewer tokens (a
+  // workspace sized for a batch serves the shorter ones): mx_proj splits T <= 64 rows of
+  // N < 8192 / slices columns, the GEMM as long as slices x its 128 x 128 tiles stay within
+  // MX_GEMM_SLICE_BLOCKS.
+  const size_t most = (size_t)128 * MX_GEMM_SLICE_BLOCKS / mx_ceil_div(N, 128);
+  const size_t want = (size_t)MX_GEMM_MAX_SLICES * T;
+  const size_t rows = want < most ? want : most;
+  return rows > (size_t)T ? rows : (size_t)T;
+}
+
+int mx_out_project(const MxDenseWork& dw, int ent, int wdt, const void* w, const void* scale,
+                   int T, int N, int K, const void* a, float* y, const float* x, float* out,
+                   hipStream_t s) {
+  const int slices = out_slices(wdt, T, N, K);
+  if (mx_proj_ok(wdt, T, K)) {
+    const MxProjSeg g{w, scale, y, N, N};
+    return mx_proj(wdt, a, T, K, &g, 1, slices, s);
+  }
+  if (mx_dense_on_gemm(wdt, T, K)) {
+    if (slices > 1) {
+      const MxGemmSeg g{w, y, N, N};
+      return mx_gemm_f16_slices(a, T, K, &g, slices, s);
+    }
+    if (!x || !out) return MX_ERR_INVALID;
+    const MxGemmSeg g{w, out, N, N, nullptr, x};
+    return mx_gemm_f16(a, T, K, &g, 1, s);
+  }
+  return mx_project(dw, ent, wdt, w, T, N, K, a, y, s);
+}
+
+int mx_out_residual(int wdt, int T, int N, int K, float* y, const float* x, float* out,
+                    hipStream_t s) {
+  const int slices = out_slices(wdt, T, N, K);
+  const bool gemm = !mx_proj_ok(wdt, T, K) && mx_dense_on_gemm(wdt, T, K);
+  if (gemm && slices == 1) return MX_OK;  // added in the GEMM's epilogue
+  const long n4 = (long)T * N / 4;
+  const dim3 grid((unsigned)((n4 + 255) / 256));
+  mx_clear_error();
+  if (slices > 1)
+    hipLaunchKernelGGL(k_residual<true>, grid, dim3(256), 0, s, x, y, n4, slices, !gemm, out);
+  else
+    hipLaunchKernelGGL(k_residual<false>, grid, dim3(256), 0, s, x, y, n4, 1, false, out);
+  return mx_launch_status();
+}
 
 size_t mx_dense_work_bytes(int T, int weight_dtype, int n_ent) {
   const int Tn = T > 0 ? T : 1;

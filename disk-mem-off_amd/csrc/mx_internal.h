@@ -143,6 +143,13 @@ struct MxGemmSeg {
 };
 // fp16 a and W.
 int mx_gemm_f16(const void* a, int M, int K, const MxGemmSeg* segs, int nseg, hipStream_t s);
+#define MX_GEMM_MAX_SLICES 8
+#define MX_GEMM_SLICE_BLOCKS 256  // blocks over which a product of few tiles is spread
+// One product with its reduction cut into `slices` (mx_gemm_f16_slice_count) slices: slice z
+// goes to y + z M n (ldy = n, no residual).
+int mx_gemm_f16_slice_count(int M, int N, int K);
+int mx_gemm_f16_slices(const void* a, int M, int K, const MxGemmSeg* seg, int slices,
+                       hipStream_t s);
 // fp32 a and W, full fp32 products; the reduction is cut into slices of kslice columns
 // (a multiple of MX_GEMM_KMULT_F32) and slice z writes its partial sums at y_s + z * yslice.
 int mx_gemm_f32_slices(const float* a, int M, int K, const MxGemmSeg* segs, int nseg,
@@ -155,8 +162,7 @@ int mx_gemm_f16x2_slices(const void* a_hi, const void* a_lo, int M, int K, const
 
 // Projections of short inputs (mx_proj.hip): fp16 or per-row int8 weights, up to
 // MX_PROJ_MAX_TOKENS tokens.  With `slices` > 1 (one segment only) the reduction is split
-// over grid slices: slice 0 goes to the segment's y, slice i to part + (i - 1) T n; the
-// residual sum adds them.
+// over grid slices: slice i is written at the segment's y + i T n.
 #define MX_PROJ_MAX_TOKENS 64
 #define MX_PROJ_MAX_SLICES 4
 struct MxProjSeg {
@@ -168,14 +174,8 @@ struct MxProjSeg {
 };
 bool mx_proj_ok(int wdt, int T, int K);
 int mx_proj_slices(int wdt, int N, int K);
-// Bytes of `part` for T tokens (does not shrink as T grows).
-size_t mx_proj_part_bytes(int wdt, int T, int N, int K);
 int mx_proj(int wdt, const void* a, int T, int K, const MxProjSeg* segs, int nseg, int slices,
-            float* part, hipStream_t s);
-// out = x + y (+ the slices in `part`; y then holds the sum) over n floats, n % 4 == 0, all
-// 16-byte aligned; out may alias x.
-int mx_residual(const float* x, float* y, const float* part, int slices, long n, float* out,
-                hipStream_t s);
+            hipStream_t s);
 
 // Workspace pieces of the dense projections of an attention block (device pointers):
 // expert-table entries (one per projection), single-group m-tile tables and ones[T] for
@@ -205,6 +205,17 @@ static inline bool mx_dense_on_gemm(int wdt, int T, int K) {
 // y[T, N] = a[T, K] W^T with W = projection `ent` (wmat, its weights, for mx_gemm_f16).
 int mx_project(const MxDenseWork& w, int ent, int wdt, const void* wmat, int T, int N, int K,
                const void* a, float* y, hipStream_t s);
+// The projection that ends an attention block, out = x + a W^T (out may alias x), in two
+// stages: the product (into y, or straight into out where the GEMM's epilogue adds x), then
+// the residual sum (nothing to do in that case).  y holds mx_out_rows(T, N) rows of N floats:
+// the reduction slices of the product follow each other there, and the sum leaves the whole
+// product in the first T rows (not written by the GEMM forms).
+size_t mx_out_rows(int T, int N);
+int mx_out_project(const MxDenseWork& dw, int ent, int wdt, const void* w, const void* scale,
+                   int T, int N, int K, const void* a, float* y, const float* x, float* out,
+                   hipStream_t s);
+int mx_out_residual(int wdt, int T, int N, int K, float* y, const float* x, float* out,
+                    hipStream_t s);
 // Chunked gated recurrence on fp32 MFMA (mx_la_chunk.hip) for key / value heads of 64 or
 // 128, with a 16-byte aligned workspace of mx_la_chunk_ws_bytes (0: shape not supported;
 // per-chunk decay coefficients and the state every chunk after the first starts from);

@@ -67,7 +67,6 @@ struct Carve {
 struct LaWork {
   MxLinearAttnViews v;
   MxDenseWork dw;      // projections: entry 0 qkvz, 1 ba, 2 out
-  float* out_part = nullptr;  // out projection of short inputs: reduction slices 1 ..
   void* chunk_ws = nullptr;  // chunked scan: coefficients and chunk states (NULL: sequential)
 };
 
@@ -89,10 +88,9 @@ int layout(const MxLinearAttnDesc* d, int T, void* ws, LaWork* w, size_t* total)
   t.v.decay = (float*)c.take(Tn * m.n * 4);
   t.v.o = (float*)c.take(Tn * m.vd * 4);
   t.v.act = c.take(Tn * m.vd * (f32 ? 4 : 2));
-  t.v.y = (float*)c.take(Tn * m.H * 4);
+  t.v.y = (float*)c.take(mx_out_rows((int)Tn, m.H) * m.H * 4);
   char* dwb = (char*)c.take(mx_dense_work_bytes((int)Tn, d->weight_dtype, 3));
   mx_dense_work_carve(dwb, (int)Tn, d->weight_dtype, 3, &t.dw);
-  t.out_part = (float*)c.take(mx_proj_part_bytes(d->weight_dtype, (int)Tn, m.H, m.vd));
   const size_t cb = mx_la_chunk_ws_bytes((int)Tn, m.n, m.dk, m.dv);
   t.chunk_ws = cb ? c.take(cb) : nullptr;
   if (w) *w = t;
@@ -666,7 +664,7 @@ int run_stage(int st, const MxLinearAttnDesc* d, const MxLinearAttnWeights* w, c
       if (mx_proj_ok(wdt, T, m.H)) {  // qkvz and ba share h: one launch
         const MxProjSeg g[2] = {{w->qkvz_w, w->qkvz_scale, k.v.qkvz, m.W1, m.W1},
                                 {w->ba_w, w->ba_scale, k.v.ba, m.W2, m.W2}};
-        return mx_proj(wdt, h, T, m.H, g, 2, 1, nullptr, s);
+        return mx_proj(wdt, h, T, m.H, g, 2, 1, s);
       }
       if (mx_dense_on_gemm(wdt, T, m.H)) {  // qkvz and ba share h: one GEMM launch
         const MxGemmSeg g[2] = {{w->qkvz_w, k.v.qkvz, m.W1, m.W1}, {w->ba_w, k.v.ba, m.W2, m.W2}};
@@ -708,22 +706,10 @@ int run_stage(int st, const MxLinearAttnDesc* d, const MxLinearAttnWeights* w, c
                            f32 ? nullptr : (half_t*)k.v.act);
       return mx_launch_status();
     case 6:
-      if (mx_proj_ok(wdt, T, m.vd)) {
-        const MxProjSeg g{w->out_w, w->out_scale, k.v.y, m.H, m.H};
-        return mx_proj(wdt, k.v.act, T, m.vd, &g, 1, mx_proj_slices(wdt, m.H, m.vd), k.out_part,
-                       s);
-      }
-      if (mx_dense_on_gemm(wdt, T, m.vd)) {  // out = x + act W_out^T in the GEMM epilogue
-        if (!x || !out) return MX_ERR_INVALID;
-        const MxGemmSeg g{w->out_w, out, m.H, m.H, nullptr, x};
-        return mx_gemm_f16(k.v.act, T, m.vd, &g, 1, s);
-      }
-      return mx_project(k.dw, 2, wdt, w->out_w, T, m.H, m.vd, k.v.act, k.v.y, s);
+      return mx_out_project(k.dw, 2, wdt, w->out_w, w->out_scale, T, m.H, m.vd, k.v.act, k.v.y, x,
+                            out, s);
     case 7:
-      if (mx_dense_on_gemm(wdt, T, m.vd)) return MX_OK;  // added in stage 6
-      return mx_residual(x, k.v.y, k.out_part,
-                         mx_proj_ok(wdt, T, m.vd) ? mx_proj_slices(wdt, m.H, m.vd) : 1,
-                         (long)T * m.H, out, s);
+      return mx_out_residual(wdt, T, m.H, m.vd, k.v.y, x, out, s);
     default:
       return MX_ERR_INVALID;
   }

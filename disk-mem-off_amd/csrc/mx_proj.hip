@@ -1,8 +1,7 @@
 // Projections of short inputs (at most MX_PROJ_MAX_TOKENS tokens): y_s[T, N_s] =
 // a[T, K] W_s[N_s, K]^T for up to MX_GEMM_MAX_SEG row-major fp16 or per-row int8 weight
 // matrices that share the fp16 activation a (linear_t, offload_runtime/executors/
-// _common.py:101-103, of the attention blocks' decode batches), and the residual sum that
-// ends those blocks.
+// _common.py:101-103, of the attention blocks' decode batches).
 //
 // Bound by the weight stream.  A block owns 16 NB output columns; its 4 waves split the
 // reduction (and, for products of few columns, up to MX_PROJ_MAX_SLICES grid slices split
@@ -39,8 +38,6 @@ struct ProjArgs {
   int unit0[MX_GEMM_MAX_SEG + 1];  // first 16 NB-column unit of each segment, then the total
   int nseg, T, K;
   const half_t* a;
-  float* part;       // slices 1 .. of the one segment's product, [T, n] each
-  long part_stride;  // floats per slice
 };
 
 template <int WF, int MT, int UB, int NB>
@@ -176,11 +173,8 @@ __global__ __launch_bounds__(256) void k_proj(const ProjArgs p) {
         r[e] *= (float)v;
       }
     }
-    float* y = blockIdx.y == 0 ? sg.y + (size_t)t * sg.ldy
-                               : p.part + (size_t)(blockIdx.y - 1) * p.part_stride +
-                                     (size_t)t * sg.n;
-    const int ld = blockIdx.y == 0 ? sg.ldy : sg.n;
-    if (n + 3 < sg.n && (ld & 3) == 0) {
+    float* y = sg.y + ((size_t)blockIdx.y * T + t) * sg.ldy;
+    if (n + 3 < sg.n && (sg.ldy & 3) == 0) {
       *(float4_t*)(y + n) = r;
     } else {
 #pragma unroll
@@ -188,28 +182,6 @@ __global__ __launch_bounds__(256) void k_proj(const ProjArgs p) {
         if (n + e < sg.n) y[n + e] = r[e];
     }
   }
-}
-
-// out = x + y (+ the further slices of y, in slice order; y then receives their sum).
-template <bool SLICED>
-__global__ __launch_bounds__(256) void k_residual(const float* x, float* y,
-                                                  const float* __restrict__ part, long stride,
-                                                  int slices, long n4, float* out) {
-  const long i = (long)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n4) return;
-  const float4_t a = ((const float4_t*)x)[i];
-  float4_t b = ((const float4_t*)y)[i];
-  if constexpr (SLICED) {
-    float4_t e[MX_PROJ_MAX_SLICES - 1];
-#pragma unroll
-    for (int s = 1; s < MX_PROJ_MAX_SLICES; ++s)
-      if (s < slices) e[s - 1] = ((const float4_t*)(part + (s - 1) * stride))[i];
-#pragma unroll
-    for (int s = 1; s < MX_PROJ_MAX_SLICES; ++s)
-      if (s < slices) b += e[s - 1];
-    ((float4_t*)y)[i] = b;
-  }
-  ((float4_t*)out)[i] = a + b;
 }
 
 template <int WF, int MT, int NB>
@@ -251,16 +223,11 @@ int mx_proj_slices(int wdt, int N, int K) {
   return s;
 }
 
-size_t mx_proj_part_bytes(int wdt, int T, int N, int K) {
-  const int t = T < MX_PROJ_MAX_TOKENS ? T : MX_PROJ_MAX_TOKENS;
-  return (size_t)(mx_proj_slices(wdt, N, K) - 1) * t * N * 4;
-}
-
 int mx_proj(int wdt, const void* a, int T, int K, const MxProjSeg* segs, int nseg, int slices,
-            float* part, hipStream_t s) {
+            hipStream_t s) {
   if (!mx_proj_ok(wdt, T, K)) return MX_ERR_UNSUPPORTED;
   if (T <= 0 || K <= 0 || !a || !segs || nseg < 1 || nseg > MX_GEMM_MAX_SEG || slices < 1 ||
-      slices > MX_PROJ_MAX_SLICES || (slices > 1 && (nseg != 1 || !part)))
+      slices > MX_PROJ_MAX_SLICES || (slices > 1 && (nseg != 1 || segs[0].ldy != segs[0].n)))
     return MX_ERR_INVALID;
   if (!mx_aligned16(a)) return MX_ERR_ALIGNMENT;
   ProjArgs p = {};
@@ -280,25 +247,11 @@ int mx_proj(int wdt, const void* a, int T, int K, const MxProjSeg* segs, int nse
   p.T = T;
   p.K = K;
   p.a = (const half_t*)a;
-  p.part = part;
-  p.part_stride = (long)T * segs[0].n;
   const int cw = mx_ceil_div(mx_ceil_div(K, chunk_cols(wdt)), 4 * slices);
   mx_clear_error();
   if (wdt == MX_DT_I8)
     launch_wf<MX_DT_I8>(p, dim3(units, slices), cw, s);
   else
     launch_wf<MX_DT_F16>(p, dim3(units, slices), cw, s);
-  return mx_launch_status();
-}
-
-int mx_residual(const float* x, float* y, const float* part, int slices, long n, float* out,
-                hipStream_t s) {
-  const long n4 = n / 4;
-  const dim3 grid((unsigned)((n4 + 255) / 256));
-  mx_clear_error();
-  if (slices > 1)
-    hipLaunchKernelGGL(k_residual<true>, grid, dim3(256), 0, s, x, y, part, n, slices, n4, out);
-  else
-    hipLaunchKernelGGL(k_residual<false>, grid, dim3(256), 0, s, x, y, nullptr, 0l, 1, n4, out);
   return mx_launch_status();
 }

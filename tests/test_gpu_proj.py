@@ -118,3 +118,54 @@ def test_full_attention_projections(mi355x, stream, wdt, T):
     _check("v", vv, h, w[fa.V])
     _check("o", y, act, w[fa.O])
     assert np.array_equal(out, x + y.astype(np.float32))
+
+
+@pytest.mark.parametrize("hidden,heads,dv,T", [
+    (192, 9, 256, 65),     # out: 36 stages in 4 slices, one row tile of 1 row past 64
+    (192, 9, 256, 129),    # two row tiles
+    (2048, 9, 64, 300),    # out: 9 stages, one slice; qkvz on two blocks per CU
+    (128, 8, 264, 128),    # out: 33 stages in 4 slices, the last one shorter
+])
+def test_linear_attention_gemm_slices(mi355x, stream, hidden, heads, dv, T):
+    shape = syn.LinearAttnShape(hidden, heads, 32, dv, 4, 1e-6)
+    print(f"[gpu] dense GEMM hidden {hidden} vd {heads * dv} T={T}", flush=True)
+    t = syn.make_linear_attn_tensors(shape, 50 + T, weight_dtype=np.float16, norm_noise=0.1)
+    w = _weights(t, (la.QKVZ, la.BA, la.OUT), "float16")
+    x = syn.make_inputs(51 + T, T, hidden)
+    layer = DeviceLinearAttnLayer.from_host(mi355x, t, stream)
+    try:
+        out = layer.forward_numpy(x, shape.eps)
+        v = layer.runner.views(layer.desc(shape.eps), T)
+
+        def read(p, dt, n):
+            return read_device(mi355x, p, dt, T * n, stream).reshape(T, n).astype(np.float64)
+
+        h, act = read(v.h16, np.float16, hidden), read(v.act, np.float16, heads * dv)
+        qkvz, ba = read(v.qkvz, np.float32, shape.qkvz_rows), read(v.ba, np.float32, shape.ba_rows)
+    finally:
+        layer.close()
+    _check("qkvz", qkvz, h, w[la.QKVZ])
+    _check("ba", ba, h, w[la.BA])
+    # out = x + act W^T: one more rounding, of a sum no larger than |x| + the magnitudes
+    wo, _ = w[la.OUT]
+    k = act.shape[1]
+    bound = ((k + 16) * 2.0 ** -24 + 2.0 ** -23) * (np.abs(act) @ np.abs(wo).T + np.abs(x)) + 1e-30
+    worst = float(np.max(np.abs(out - (x + act @ wo.T)) / bound))
+    print(f"    out K={k}: worst error {worst:.3f} of the bound", flush=True)
+    assert worst <= 1.0
+
+
+def test_workspace_never_shrinks_with_tokens(mi355x):
+    """A workspace sized for a batch serves every shorter one (the executors size it once)."""
+    from moe_mi355x import _lib
+    from moe_mi355x.full_attn import workspace_bytes as fa_bytes
+    from moe_mi355x.linear_attn import workspace_bytes as la_bytes
+
+    for wdt in (_lib.MX_DT_F32, _lib.MX_DT_F16, _lib.MX_DT_I8):
+        for hidden, n, dk, dv in ((2048, 32, 128, 128), (192, 9, 32, 256), (8192, 4, 64, 64)):
+            d = _lib.MxLinearAttnDesc(hidden, n, dk, dv, 4, wdt, _lib.MX_DT_F32, 1e-6)
+            sizes = [la_bytes(d, T) for T in range(1, 700)]
+            assert sizes == sorted(sizes)
+            f = _lib.MxFullAttnDesc(hidden, n, 1, dk, dk // 2, wdt, _lib.MX_DT_F32, 1e4, 1e-6)
+            sizes = [fa_bytes(f, T) for T in range(1, 700)]
+            assert sizes == sorted(sizes)
