@@ -1,11 +1,14 @@
 // Dense GEMM on MFMA with an LDS-staged operand ring:
 //   y_s[M, N_s] (fp32, row stride ldy_s) = a[M, K] . W_s[N_s, K]^T
 // for up to MX_GEMM_MAX_SEG weight matrices W_s (nn.Linear row-major) that share the
-// activations a.  Two element types:
+// activations a.  Element types:
 //  * fp16 operands (v_mfma_f32_16x16x32_f16): the long-input projections of the attention
 //    blocks (the q / k / v projections, or qkvz and ba, in one launch).  Reference:
 //    linear_t = x @ W.T (offload_runtime/executors/_common.py:101-103) at
 //    qwen3_next.py:170-174, :211, :231, :245 and :268.
+//  * fp16 activations and per-row int8 weights, for the same projections: the weights stay
+//    int8 up to the operand registers, where 16 of them become two fp16 fragments (exact,
+//    the conversion of the expert kernels); the row scale multiplies the finished sums;
 //  * fp32 operands (v_mfma_f32_16x16x4_f32, full fp32 products), and
 //  * fp32 operands carried as two fp16 planes each (SPLIT): x = hi + 2^-11 lo with
 //    hi = fp16(x), lo = fp16((x - hi) * 2^11), and a . w = a_hi . w_hi + 2^-11 (a_hi . w_lo
@@ -57,6 +60,7 @@ __device__ __forceinline__ rsrc_t make_rsrc(const void* base, uint32_t bytes) {
 struct GemmSeg {
   const void* w;  // [N, K]
   const void* w_lo;  // SPLIT: the low plane of w
+  const void* scale;  // I8: fp16 scale of each weight row
   const float* res;  // residual added by the epilogue (same layout as y) or null
   float* y;       // [M, ldy] for slice 0; slice z at y + z * yslice
   int n;          // N of the segment
@@ -95,19 +99,27 @@ __device__ __forceinline__ int gemm_read_pos(int j, int q, int ks) {
   return (j >> 3) * 1024 + (j & 7) * 128 + ((((ks << 2) + q) ^ (j & 7)) << 4);
 }
 
-template <typename ET, bool SPLIT, int BM, int BN, int WM, int WN, int NS, int OCC>
+// Operand forms of the kernel: both operands of ET; both as two fp16 planes; fp16
+// activations and per-row int8 weights.
+enum GemmForm { PLAIN, SPLIT2, I8W };
+
+template <typename ET, int FORM, int BM, int BN, int WM, int WN, int NS, int OCC>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, OCC) void k_gemm_nt(
     const GemmArgs p) {
   constexpr int ES = sizeof(ET);
   constexpr int NWN = BN / WN, NW = (BM / WM) * NWN;
   constexpr int MF = WM / 16, NF = WN / 16;
-  constexpr int PL = SPLIT ? 2 : 1;               // planes per operand
+  constexpr bool SPLIT = FORM == SPLIT2, I8 = FORM == I8W;
+  // Planes per operand and stage slot.  I8: a stage is 128 reduction columns, one 128-byte
+  // piece of each weight row and two of each activation row, in a plane each.
+  constexpr int PL = SPLIT ? 2 : 1, PLA = FORM == PLAIN ? 1 : 2;
+  constexpr int KST = I8 ? STAGE_BYTES : STAGE_BYTES / ES;   // reduction columns per stage
   constexpr int FA1 = BM / FRAG_ROWS, FB1 = BN / FRAG_ROWS;  // fragments per plane and stage
-  constexpr int FA = PL * FA1, FT = FA + PL * FB1;  // fragments per stage slot: A planes, B planes
+  constexpr int FA = PLA * FA1, FT = FA + PL * FB1;  // fragments per stage slot: A planes, B planes
   constexpr int SLOT = FT * 1024;
   constexpr int PA = BM * STAGE_BYTES, PB = BN * STAGE_BYTES;  // bytes of one plane per slot
   constexpr int DPW = FT / NW;                    // copies per wave and stage
-  static_assert(!SPLIT || ES == 2, "split planes are fp16");
+  static_assert(FORM == PLAIN || ES == 2, "split planes and the activations of I8 are fp16");
   static_assert(FA1 % NW == 0 && FB1 % NW == 0, "fragments must divide among the waves");
   static_assert(NS >= 2, "a stage ring of at least two slots");
   __shared__ __align__(1024) char lds[NS * SLOT];
@@ -153,7 +165,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, OCC) void k_gemm_nt(
   const int j = lane & 15, q = lane >> 4;
 
   const rsrc_t ra = make_rsrc(p.a, (uint32_t)((size_t)M * K * ES));
-  const rsrc_t rb = make_rsrc(sg.w, (uint32_t)((size_t)N * K * ES));
+  const rsrc_t rb = make_rsrc(sg.w, (uint32_t)((size_t)N * K * (I8 ? 1 : ES)));
   const rsrc_t ral = SPLIT ? make_rsrc(p.a_lo, (uint32_t)((size_t)M * K * ES)) : ra;
   const rsrc_t rbl = SPLIT ? make_rsrc(sg.w_lo, (uint32_t)((size_t)N * K * ES)) : rb;
   // Fragment f of a slot: A planes [0, FA) (plane f / FA1), then B planes (plane
@@ -162,7 +174,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, OCC) void k_gemm_nt(
   auto rsrc_of = [&](int i) {
     const int f0 = i * NW;
     if (f0 < FA1) return ra;
-    if (f0 < FA) return ral;
+    if (f0 < FA) return SPLIT ? ral : ra;
     if (f0 < FA + FB1) return rb;
     return rbl;
   };
@@ -175,10 +187,11 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, OCC) void k_gemm_nt(
     const int f = wave + i * NW;
     if (i * NW < FA) {
       const int row = m0 + FRAG_ROWS * (f % FA1) + cr;
-      goff[i] = row < M ? ((uint32_t)row * (uint32_t)K + k0) * ES + cq * 16 : kOob;
+      const int piece = I8 ? i * NW / FA1 * STAGE_BYTES : 0;  // the plane's part of the stage
+      goff[i] = row < M ? ((uint32_t)row * (uint32_t)K + k0) * ES + piece + cq * 16 : kOob;
     } else {
       const int row = n0 + FRAG_ROWS * ((f - FA) % FB1) + cr;
-      goff[i] = row < N ? ((uint32_t)row * (uint32_t)K + k0) * ES + cq * 16 : kOob;
+      goff[i] = row < N ? ((uint32_t)row * (uint32_t)K + k0) * (I8 ? 1 : ES) + cq * 16 : kOob;
     }
   }
   // K and the slice length are multiples of the stage width, so every piece of a stage lies
@@ -189,7 +202,8 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, OCC) void k_gemm_nt(
 #pragma unroll
     for (int i = 0; i < DPW; ++i) {
       const int f = wave + i * NW;
-      mx_copy_to_lds16(rsrc_of(i), slot + f * 1024, goff[i] + (uint32_t)st * STAGE_BYTES);
+      const uint32_t step = I8 && i * NW < FA ? 2 * STAGE_BYTES : STAGE_BYTES;
+      mx_copy_to_lds16(rsrc_of(i), slot + f * 1024, goff[i] + (uint32_t)st * step);
     }
   };
 
@@ -212,7 +226,14 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, OCC) void k_gemm_nt(
 #pragma unroll
   for (int ks = 0; ks < KSTEPS; ++ks) rpos[ks] = gemm_read_pos(j, q, ks);
 
-  const int nst = kn / (STAGE_BYTES / ES);
+  // I8: the k-step pair ks (64 columns) takes 16 columns per lane, 64 ks + 16 q .., of both
+  // operands: one weight piece, and the activation pieces 2 q and 2 q + 1 of plane ks.
+  int apos[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+    apos[h] = (j >> 3) * 1024 + (j & 7) * 128 + (((2 * q + h) ^ (j & 7)) << 4);
+
+  const int nst = kn / KST;
 #pragma unroll
   for (int s0 = 0; s0 < NS - 1; ++s0)
     if (s0 < nst) issue(s0);
@@ -229,6 +250,27 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, OCC) void k_gemm_nt(
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks) {
       int4_t af[MF], bf[NF];
+      if constexpr (I8) {
+        half8_t w[2][NF];
+#pragma unroll
+        for (int ni = 0; ni < NF; ++ni)
+          bf[ni] = *(const int4_t*)(slot + PLA * PA + (wn * NF + ni) * BLK16 + rpos[ks]);
+#pragma unroll
+        for (int ni = 0; ni < NF; ++ni) mx_i8_to_f16(bf[ni], w[0][ni], w[1][ni]);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+          for (int mi = 0; mi < MF; ++mi)
+            af[mi] = *(const int4_t*)(slot + ks * PA + (wm * MF + mi) * BLK16 + apos[h]);
+#pragma unroll
+          for (int mi = 0; mi < MF; ++mi)
+#pragma unroll
+            for (int ni = 0; ni < NF; ++ni)
+              acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                  w[h][ni], __builtin_bit_cast(half8_t, af[mi]), acc[mi][ni], 0, 0, 0);
+        }
+        continue;
+      }
 #pragma unroll
       for (int mi = 0; mi < MF; ++mi)
         af[mi] = *(const int4_t*)(slot + (wm * MF + mi) * BLK16 + rpos[ks]);
@@ -287,6 +329,20 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, OCC) void k_gemm_nt(
           acc[mi][ni][r] = fmaf(acc2[mi][ni][r], 1.f / 2048.f, acc[mi][ni][r]);
   }
 
+  if constexpr (I8) {
+#pragma unroll
+    for (int ni = 0; ni < NF; ++ni) {
+      float sc[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        sc[r] = (float)((const half_t*)sg.scale)[min(n0 + wn * WN + ni * 16 + 4 * q + r, N - 1)];
+#pragma unroll
+      for (int mi = 0; mi < MF; ++mi)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[mi][ni][r] *= sc[r];
+    }
+  }
+
   // Epilogue: fp32 rows of the segment's output, 4 consecutive columns per lane (a
   // 16-byte store when the row stride and the base allow it), plus the residual when the
   // segment has one (read and written by the same lane, so it may alias the output).
@@ -341,7 +397,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, OCC) void k_gemm_nt(
   }
 }
 
-template <typename ET, bool SPLIT, int BM, int BN, int WM, int WN, int NS, int OCC>
+template <typename ET, int FORM, int BM, int BN, int WM, int WN, int NS, int OCC>
 int launch(GemmArgs& args, const MxGemmSeg* segs, int nseg, int splits, hipStream_t s) {
   args.mblk = mx_ceil_div(args.M, BM);
   long blocks = 0;
@@ -353,17 +409,18 @@ int launch(GemmArgs& args, const MxGemmSeg* segs, int nseg, int splits, hipStrea
     return MX_ERR_UNSUPPORTED;
   constexpr int threads = (BM / WM) * (BN / WN) * 64;
   mx_clear_error();
-  hipLaunchKernelGGL((k_gemm_nt<ET, SPLIT, BM, BN, WM, WN, NS, OCC>), dim3((unsigned)blocks, splits),
+  hipLaunchKernelGGL((k_gemm_nt<ET, FORM, BM, BN, WM, WN, NS, OCC>), dim3((unsigned)blocks, splits),
                      dim3(threads), 0, s, args);
   return mx_launch_status();
 }
 
-// Shared argument checks; fills args (segments, K, slices) for element size es.
-int prepare(GemmArgs& args, const void* a, int M, int K, int es, const MxGemmSeg* segs,
+// Shared argument checks; fills args (segments, K, slices) for activations of element size
+// es and weights of size wes.
+int prepare(GemmArgs& args, const void* a, int M, int K, int es, int wes, const MxGemmSeg* segs,
             int nseg, int kslice, long yslice) {
   if (!a || !segs || nseg < 1 || nseg > MX_GEMM_MAX_SEG || M <= 0 || K <= 0 || kslice <= 0)
     return MX_ERR_INVALID;
-  const int bke = STAGE_BYTES / es;
+  const int bke = STAGE_BYTES / wes;
   if (K % bke || kslice % bke) return MX_ERR_UNSUPPORTED;  // whole stages only
   if (!mx_aligned16(a)) return MX_ERR_ALIGNMENT;
   if ((long)M * K * es >= (1l << 31)) return MX_ERR_UNSUPPORTED;
@@ -379,9 +436,11 @@ int prepare(GemmArgs& args, const void* a, int M, int K, int es, const MxGemmSeg
     if (!g.w || !g.y || g.n <= 0 || g.ldy < g.n) return MX_ERR_INVALID;
     if (g.res && kslice != K) return MX_ERR_INVALID;  // a residual needs the whole reduction
     if (!mx_aligned16(g.w)) return MX_ERR_ALIGNMENT;
-    if ((long)g.n * K * es >= (1l << 31)) return MX_ERR_UNSUPPORTED;
+    if (wes == 1 && !g.scale) return MX_ERR_INVALID;
+    if ((long)g.n * K * wes >= (1l << 31)) return MX_ERR_UNSUPPORTED;
     args.seg[i].w = g.w;
     args.seg[i].w_lo = g.w_lo;
+    args.seg[i].scale = g.scale;
     args.seg[i].res = g.res;
     args.seg[i].y = g.y;
     args.seg[i].n = g.n;
@@ -397,14 +456,27 @@ int prepare(GemmArgs& args, const void* a, int M, int K, int es, const MxGemmSeg
 // v: 27.4 and 26.9); with more blocks than CUs two blocks per CU with two slots each (q + k +
 // v of 777 tokens, 504 blocks: 54 -> 41 us, of 1500 tokens 99 -> 74; qkvz + ba of 300 tokens
 // 54 -> 44.6, of 1000 tokens 157 -> 122 us, against rounds of one block per CU).
-int launch_small(GemmArgs& args, const MxGemmSeg* segs, int nseg, int splits, hipStream_t s) {
+int launch_small(int wdt, GemmArgs& args, const MxGemmSeg* segs, int nseg, int splits,
+                 hipStream_t s) {
+  // int8: stages of 128 columns, 48 KiB, one block per CU.
+  if (wdt == MX_DT_I8)
+    return launch<half_t, I8W, 128, 128, 64, 32, 3, 1>(args, segs, nseg, splits, s);
   long blocks = 0;
   for (int i = 0; i < nseg; ++i)
     blocks += (long)mx_ceil_div(args.M, 128) * mx_ceil_div(segs[i].n, 128);
   if (blocks * splits > 256)
-    return launch<half_t, false, 128, 128, 64, 64, 2, 2>(args, segs, nseg, splits, s);
-  return launch<half_t, false, 128, 128, 64, 32, 4, 1>(args, segs, nseg, splits, s);
+    return launch<half_t, PLAIN, 128, 128, 64, 64, 2, 2>(args, segs, nseg, splits, s);
+  return launch<half_t, PLAIN, 128, 128, 64, 32, 4, 1>(args, segs, nseg, splits, s);
 }
+
+// Tiles of 256 columns: 256 rows for fp16 weights; 128 rows, as many bytes per product, for
+// int8.
+int launch_big(int wdt, GemmArgs& args, const MxGemmSeg* segs, int nseg, hipStream_t s) {
+  if (wdt == MX_DT_I8) return launch<half_t, I8W, 128, 256, 64, 64, 2, 1>(args, segs, nseg, 1, s);
+  return launch<half_t, PLAIN, 256, 256, 128, 64, 2, 1>(args, segs, nseg, 1, s);
+}
+
+int stage_cols(int wdt) { return wdt == MX_DT_I8 ? STAGE_BYTES : MX_GEMM_KMULT_F16; }
 
 }  // namespace
 
@@ -412,27 +484,27 @@ int launch_small(GemmArgs& args, const MxGemmSeg* segs, int nseg, int splits, hi
 // that the tiles times the slices fill the CUs once: 2048 columns over 4096, 100 tokens 43.5
 // -> 10 us with 8 slices, 300 tokens 44.5 -> 15 with 5, 777 tokens 48 -> 27.8 with 2 (and
 // 4-7 us for the launch that adds the slices and x).  Two blocks per CU (512) gained nothing
-// below 1500 tokens (300: 17.0 + 8.4 us; 777: 25.9 + 9.1).  A slice keeps at least 8 stages.
-int mx_gemm_f16_slice_count(int M, int N, int K) {
+// below 1500 tokens (300: 17.0 + 8.4 us; 777: 25.9 + 9.1).  A slice keeps at least 512
+// columns, and the last one (the slices before it are equally long) at least one stage.
+int mx_gemm_slice_count(int wdt, int M, int N, int K) {
   const int blocks = mx_ceil_div(M, 128) * mx_ceil_div(N, 128);
-  const int nst = K / MX_GEMM_KMULT_F16;
   int s = MX_GEMM_SLICE_BLOCKS / blocks;
   if (s > MX_GEMM_MAX_SLICES) s = MX_GEMM_MAX_SLICES;
-  while (s > 1 && nst / s < 8) --s;
+  const int nst = K / stage_cols(wdt);
+  while (s > 1 && (K / s < 512 || (s - 1) * mx_ceil_div(nst, s) >= nst)) --s;
   return s < 1 ? 1 : s;
 }
 
-int mx_gemm_f16_slices(const void* a, int M, int K, const MxGemmSeg* seg, int slices,
-                       hipStream_t s) {
+int mx_gemm_slices(int wdt, const void* a, int M, int K, const MxGemmSeg* seg, int slices,
+                   hipStream_t s) {
   if (!seg || slices < 1 || slices > MX_GEMM_MAX_SLICES || seg->ldy != seg->n || seg->res)
     return MX_ERR_INVALID;
-  const int nst = K / MX_GEMM_KMULT_F16;
-  // Slices of equal length but the last, every one with at least one stage.
+  const int kc = stage_cols(wdt), nst = K / kc;
   const int per = mx_ceil_div(nst, slices);
   if (nst < 1 || (slices - 1) * per >= nst) return MX_ERR_INVALID;
   GemmArgs args;
-  MX_TRY(prepare(args, a, M, K, 2, seg, 1, per * MX_GEMM_KMULT_F16, (long)M * seg->n));
-  return launch_small(args, seg, 1, slices, s);
+  MX_TRY(prepare(args, a, M, K, 2, wdt == MX_DT_I8 ? 1 : 2, seg, 1, per * kc, (long)M * seg->n));
+  return launch_small(wdt, args, seg, 1, slices, s);
 }
 
 #ifndef MX_GEMM_MID
@@ -442,29 +514,39 @@ int mx_gemm_f16_slices(const void* a, int M, int K, const MxGemmSeg* seg, int sl
 #define MX_GEMM_TAIL 1  // leftover columns of a partial last round on 128 x 128 tiles
 #endif
 
-int mx_gemm_f16(const void* a, int M, int K, const MxGemmSeg* segs, int nseg, hipStream_t s) {
+int mx_gemm(int wdt, const void* a, int M, int K, const MxGemmSeg* segs, int nseg,
+            hipStream_t s) {
+  const int wes = wdt == MX_DT_I8 ? 1 : 2;
   GemmArgs args;
-  MX_TRY(prepare(args, a, M, K, 2, segs, nseg, K, 0));
+  MX_TRY(prepare(args, a, M, K, 2, wes, segs, nseg, K, 0));
   long cols = 0;
   for (int i = 0; i < nseg; ++i) cols += segs[i].n;
-  // 256 x 256 tiles while they give at least two rounds of blocks on 256 CUs; 128 x 128
-  // otherwise.
-  const long big = (long)mx_ceil_div(M, 256) * mx_ceil_div((int)cols, 256);
-  if (big < 512) {
-    // 256 x 128 tiles (8 waves of 64 x 64, one block per CU) when they fill whole rounds
+  const int mblk = mx_ceil_div(M, wdt == MX_DT_I8 ? 128 : 256);
+  const long big = (long)mblk * mx_ceil_div((int)cols, 256);
+  if (wdt == MX_DT_I8) {
+    // 128 x 256 tiles once 128 x 128 ones would not fit one round: a 2048-column reduction
+    // takes 42 us a round on the large tiles, 25 on the small ones (qkvz + ba of 300 tokens, 243
+    // against 483 blocks: 50 -> 42 us).  128 x 64 and 64 x 128 tiles at two blocks per CU
+    // matched the 128 x 128 ones (48-53 us).
+    long small = 0;
+    for (int i = 0; i < nseg; ++i) small += (long)mblk * mx_ceil_div(segs[i].n, 128);
+    if (small <= 256) return launch_small(wdt, args, segs, nseg, 1, s);
+  } else if (big < 512) {
+    // 256 x 256 tiles while they give at least two rounds of blocks on 256 CUs; else 256 x 128
+    // (8 waves of 64 x 64, one block per CU) when they fill whole rounds, else 128 x 128.
     long mid = 0;
-    for (int i = 0; i < nseg; ++i) mid += (long)mx_ceil_div(M, 256) * mx_ceil_div(segs[i].n, 128);
+    for (int i = 0; i < nseg; ++i) mid += (long)mblk * mx_ceil_div(segs[i].n, 128);
     if (MX_GEMM_MID && mid >= 256 && mid % 256 == 0)
-      return launch<half_t, false, 256, 128, 64, 64, 3, 1>(args, segs, nseg, 1, s);
-    return launch_small(args, segs, nseg, 1, s);
+      return launch<half_t, PLAIN, 256, 128, 64, 64, 3, 1>(args, segs, nseg, 1, s);
+    return launch_small(wdt, args, segs, nseg, 1, s);
   }
-  if (MX_GEMM_TAIL && big % 256) {
-    // One 256 x 256 block per CU: the blocks past the last whole round would run as a
-    // partial round as long as a full one.  The whole rounds take whole 256-column tiles
-    // of the segments in order; the columns left over (partial tiles, later segments) go
-    // to a second launch on 128 x 128 tiles, which spreads them over all CUs.  Each output
+  if (MX_GEMM_TAIL && big > 256 && big % 256) {
+    // One big block per CU: the blocks past the last whole round would run as a partial
+    // round as long as a full one.  The whole rounds take whole 256-column tiles of the
+    // segments in order; the columns left over (partial tiles, later segments) go to a
+    // second launch on 128 x 128 tiles, which spreads them over all CUs.  Each output
     // element is still computed by one block over the whole reduction.
-    int budget = (int)(big / 256 * 256 / mx_ceil_div(M, 256));  // 256-column tiles
+    int budget = (int)(big / 256 * 256 / mblk);  // 256-column tiles
     MxGemmSeg head[MX_GEMM_MAX_SEG], tail[MX_GEMM_MAX_SEG];
     int nh = 0, nt = 0;
     for (int i = 0; i < nseg; ++i) {
@@ -478,7 +560,8 @@ int mx_gemm_f16(const void* a, int M, int K, const MxGemmSeg* segs, int nseg, hi
       }
       if (n0 < g.n) {
         MxGemmSeg t = g;
-        t.w = (const char*)g.w + (size_t)n0 * K * 2;
+        t.w = (const char*)g.w + (size_t)n0 * K * wes;
+        if (g.scale) t.scale = (const half_t*)g.scale + n0;
         t.y = g.y + n0;
         if (g.res) t.res = g.res + n0;
         t.n = g.n - n0;
@@ -487,28 +570,28 @@ int mx_gemm_f16(const void* a, int M, int K, const MxGemmSeg* segs, int nseg, hi
     }
     if (nh > 0 && nt > 0) {
       GemmArgs ah, at;
-      MX_TRY(prepare(ah, a, M, K, 2, head, nh, K, 0));
-      MX_TRY(prepare(at, a, M, K, 2, tail, nt, K, 0));
-      MX_TRY((launch<half_t, false, 256, 256, 128, 64, 2, 1>(ah, head, nh, 1, s)));
-      return launch_small(at, tail, nt, 1, s);
+      MX_TRY(prepare(ah, a, M, K, 2, wes, head, nh, K, 0));
+      MX_TRY(prepare(at, a, M, K, 2, wes, tail, nt, K, 0));
+      MX_TRY(launch_big(wdt, ah, head, nh, s));
+      return launch_small(wdt, at, tail, nt, 1, s);
     }
   }
-  return launch<half_t, false, 256, 256, 128, 64, 2, 1>(args, segs, nseg, 1, s);
+  return launch_big(wdt, args, segs, nseg, s);
 }
 
 int mx_gemm_f32_slices(const float* a, int M, int K, const MxGemmSeg* segs, int nseg,
                        int kslice, long yslice, hipStream_t s) {
   GemmArgs args;
-  MX_TRY(prepare(args, a, M, K, 4, segs, nseg, kslice, yslice));
+  MX_TRY(prepare(args, a, M, K, 4, 4, segs, nseg, kslice, yslice));
   const int splits = mx_ceil_div(K, kslice);
   if (splits > 1 && yslice <= 0) return MX_ERR_INVALID;
-  return launch<float, false, 128, 128, 64, 64, 2, 2>(args, segs, nseg, splits, s);
+  return launch<float, PLAIN, 128, 128, 64, 64, 2, 2>(args, segs, nseg, splits, s);
 }
 
 int mx_gemm_f16x2_slices(const void* a_hi, const void* a_lo, int M, int K, const MxGemmSeg* segs,
                          int nseg, int kslice, long yslice, hipStream_t s) {
   GemmArgs args;
-  MX_TRY(prepare(args, a_hi, M, K, 2, segs, nseg, kslice, yslice));
+  MX_TRY(prepare(args, a_hi, M, K, 2, 2, segs, nseg, kslice, yslice));
   if (!a_lo || !mx_aligned16(a_lo)) return a_lo ? MX_ERR_ALIGNMENT : MX_ERR_INVALID;
   for (int i = 0; i < nseg; ++i) {
     if (!segs[i].w_lo) return MX_ERR_INVALID;
@@ -518,6 +601,6 @@ int mx_gemm_f16x2_slices(const void* a_hi, const void* a_lo, int M, int K, const
   const int splits = mx_ceil_div(K, kslice);
   if (splits > 1 && yslice <= 0) return MX_ERR_INVALID;
   // 128 x 128 tiles of 8 waves (64 x 32 each), one block per CU (two 64 KiB stage slots).
-  return launch<half_t, true, MX_GEMM_SPLIT_BM, MX_GEMM_SPLIT_BN, 64, 32, 2, 1>(args, segs, nseg,
+  return launch<half_t, SPLIT2, MX_GEMM_SPLIT_BM, MX_GEMM_SPLIT_BN, 64, 32, 2, 1>(args, segs, nseg,
                                                                                splits, s);
 }

@@ -1,6 +1,7 @@
 // Dense projections of the attention blocks: y[T, N] = a[T, K] W^T on the single-group
-// down-projection kernels of the MoE experts (short inputs, and int8 / fp32 weights at any
-// length) or on the dense fp16 MFMA GEMM (mx_gemm_f16, long inputs with fp16 weights).
+// down-projection kernels of the MoE experts (fp32 weights, and reduction lengths that the
+// others do not take), and the projection that ends an attention block, on whichever of
+// mx_proj (short inputs), mx_gemm (long ones) and those kernels runs it.
 #include "mx_common.h"
 #include "mx_internal.h"
 
@@ -55,7 +56,7 @@ static_assert(MX_PROJ_MAX_SLICES <= MX_GEMM_MAX_SLICES, "k_residual adds either'
 // Reduction slices of an output projection.
 int out_slices(int wdt, int T, int N, int K) {
   if (mx_proj_ok(wdt, T, K)) return mx_proj_slices(wdt, N, K);
-  if (mx_dense_on_gemm(wdt, T, K)) return mx_gemm_f16_slice_count(T, N, K);
+  if (mx_dense_on_gemm(wdt, T, K)) return mx_gemm_slice_count(wdt, T, N, K);
   return 1;
 }
 
@@ -82,14 +83,14 @@ int mx_out_project(const MxDenseWork& dw, int ent, int wdt, const void* w, const
   }
   if (mx_dense_on_gemm(wdt, T, K)) {
     if (slices > 1) {
-      const MxGemmSeg g{w, y, N, N};
-      return mx_gemm_f16_slices(a, T, K, &g, slices, s);
+      const MxGemmSeg g{w, y, N, N, nullptr, nullptr, scale};
+      return mx_gemm_slices(wdt, a, T, K, &g, slices, s);
     }
     if (!x || !out) return MX_ERR_INVALID;
-    const MxGemmSeg g{w, out, N, N, nullptr, x};
-    return mx_gemm_f16(a, T, K, &g, 1, s);
+    const MxGemmSeg g{w, out, N, N, nullptr, x, scale};
+    return mx_gemm(wdt, a, T, K, &g, 1, s);
   }
-  return mx_project(dw, ent, wdt, w, T, N, K, a, y, s);
+  return mx_project(dw, ent, wdt, T, N, K, a, y, s);
 }
 
 int mx_out_residual(int wdt, int T, int N, int K, float* y, const float* x, float* out,
@@ -142,13 +143,9 @@ int mx_dense_setup(const MxDenseWork& w, const MxDenseEntries& ents, int T, hipS
   return mx_launch_status();
 }
 
-int mx_project(const MxDenseWork& w, int ent, int wdt, const void* wmat, int T, int N, int K,
-               const void* a, float* y, hipStream_t s) {
+int mx_project(const MxDenseWork& w, int ent, int wdt, int T, int N, int K, const void* a,
+               float* y, hipStream_t s) {
   if (ent < 0 || ent >= w.n_ent) return MX_ERR_INVALID;
-  if (mx_dense_on_gemm(wdt, T, K)) {
-    const MxGemmSeg g{wmat, y, N, N};
-    return mx_gemm_f16(a, T, K, &g, 1, s);
-  }
   const MxDenseTables tab{w.tabs + 0, w.tabs + 1, w.tabs + 2, w.mt_group, w.mt_row0,
                           w.tabs + 3, w.ones, w.m_blk};
   return mx_dense_linear(wdt, 0, w.entries + ent, tab, T, N, K, a, y, s);

@@ -132,6 +132,7 @@ int mx_dense_linear(int wdt, int tiled, const MxExpertPtrs* entry, const MxDense
 #define MX_GEMM_MAX_SEG 3
 #define MX_GEMM_STAGE_BYTES 128
 #define MX_GEMM_KMULT_F16 (MX_GEMM_STAGE_BYTES / 2)
+#define MX_GEMM_KMULT_I8 MX_GEMM_STAGE_BYTES
 #define MX_GEMM_KMULT_F32 (MX_GEMM_STAGE_BYTES / 4)
 struct MxGemmSeg {
   const void* w;  // [n, K] row-major (16-byte aligned), element type of a
@@ -139,17 +140,19 @@ struct MxGemmSeg {
   int n;
   int ldy;
   const void* w_lo = nullptr;  // mx_gemm_f16x2_slices: the low fp16 plane of w
-  const float* res = nullptr;  // mx_gemm_f16: y = res + a W^T (res [M, ldy], may alias y)
+  const float* res = nullptr;  // mx_gemm: y = res + a W^T (res [M, ldy], may alias y)
+  const void* scale = nullptr;  // int8 W: fp16 scale of each row
 };
-// fp16 a and W.
-int mx_gemm_f16(const void* a, int M, int K, const MxGemmSeg* segs, int nseg, hipStream_t s);
+// fp16 a; W fp16 or per-row int8 (wdt), K a multiple of MX_GEMM_KMULT_F16 / MX_GEMM_KMULT_I8.
+int mx_gemm(int wdt, const void* a, int M, int K, const MxGemmSeg* segs, int nseg,
+            hipStream_t s);
+// One product with its reduction cut into `slices` (mx_gemm_slice_count) slices: slice z goes
+// to y + z M n (ldy = n, no residual).
 #define MX_GEMM_MAX_SLICES 8
 #define MX_GEMM_SLICE_BLOCKS 256  // blocks over which a product of few tiles is spread
-// One product with its reduction cut into `slices` (mx_gemm_f16_slice_count) slices: slice z
-// goes to y + z M n (ldy = n, no residual).
-int mx_gemm_f16_slice_count(int M, int N, int K);
-int mx_gemm_f16_slices(const void* a, int M, int K, const MxGemmSeg* seg, int slices,
-                       hipStream_t s);
+int mx_gemm_slice_count(int wdt, int M, int N, int K);
+int mx_gemm_slices(int wdt, const void* a, int M, int K, const MxGemmSeg* seg, int slices,
+                   hipStream_t s);
 // fp32 a and W, full fp32 products; the reduction is cut into slices of kslice columns
 // (a multiple of MX_GEMM_KMULT_F32) and slice z writes its partial sums at y_s + z * yslice.
 int mx_gemm_f32_slices(const float* a, int M, int K, const MxGemmSeg* segs, int nseg,
@@ -179,7 +182,7 @@ int mx_proj(int wdt, const void* a, int T, int K, const MxProjSeg* segs, int nse
 
 // Workspace pieces of the dense projections of an attention block (device pointers):
 // expert-table entries (one per projection), single-group m-tile tables and ones[T] for
-// the grouped-GEMM kernels.  Long inputs with fp16 weights run on mx_gemm_f16 instead.
+// the grouped-GEMM kernels, for what neither mx_proj nor mx_gemm takes.
 #define MX_DENSE_GEMM_MIN_TOKENS 65
 #define MX_DENSE_MAX_ENT 4
 struct MxDenseEntries {
@@ -198,13 +201,14 @@ void mx_dense_work_carve(char* base, int T, int weight_dtype, int n_ent, MxDense
 // Writes the table entries and m-tile tables (one small launch per block call).
 int mx_dense_setup(const MxDenseWork& w, const MxDenseEntries& ents, int T, hipStream_t s);
 // Whether projections of T tokens with these weights and reduction length K run on
-// mx_gemm_f16 (fp16 weights, long inputs, K a multiple of its stage width).
+// mx_gemm (fp16 or int8 weights, long inputs, K a multiple of its stage width).
 static inline bool mx_dense_on_gemm(int wdt, int T, int K) {
-  return wdt == MX_DT_F16 && T >= MX_DENSE_GEMM_MIN_TOKENS && K % MX_GEMM_KMULT_F16 == 0;
+  return T >= MX_DENSE_GEMM_MIN_TOKENS && ((wdt == MX_DT_F16 && K % MX_GEMM_KMULT_F16 == 0) ||
+                                           (wdt == MX_DT_I8 && K % MX_GEMM_KMULT_I8 == 0));
 }
-// y[T, N] = a[T, K] W^T with W = projection `ent` (wmat, its weights, for mx_gemm_f16).
-int mx_project(const MxDenseWork& w, int ent, int wdt, const void* wmat, int T, int N, int K,
-               const void* a, float* y, hipStream_t s);
+// y[T, N] = a[T, K] W^T with W = projection `ent`, on the grouped kernels.
+int mx_project(const MxDenseWork& w, int ent, int wdt, int T, int N, int K, const void* a,
+               float* y, hipStream_t s);
 // The projection that ends an attention block, out = x + a W^T (out may alias x), in two
 // stages: the product (into y, or straight into out where the GEMM's epilogue adds x), then
 // the residual sum (nothing to do in that case).  y holds mx_out_rows(T, N) rows of N floats:

@@ -667,13 +667,15 @@ int run_stage(int st, const MxLinearAttnDesc* d, const MxLinearAttnWeights* w, c
         return mx_proj(wdt, h, T, m.H, g, 2, 1, s);
       }
       if (mx_dense_on_gemm(wdt, T, m.H)) {  // qkvz and ba share h: one GEMM launch
-        const MxGemmSeg g[2] = {{w->qkvz_w, k.v.qkvz, m.W1, m.W1}, {w->ba_w, k.v.ba, m.W2, m.W2}};
-        return mx_gemm_f16(h, T, m.H, g, 2, s);
+        const MxGemmSeg g[2] = {
+            {w->qkvz_w, k.v.qkvz, m.W1, m.W1, nullptr, nullptr, w->qkvz_scale},
+            {w->ba_w, k.v.ba, m.W2, m.W2, nullptr, nullptr, w->ba_scale}};
+        return mx_gemm(wdt, h, T, m.H, g, 2, s);
       }
-      return mx_project(k.dw, 0, wdt, w->qkvz_w, T, m.W1, m.H, h, k.v.qkvz, s);
+      return mx_project(k.dw, 0, wdt, T, m.W1, m.H, h, k.v.qkvz, s);
     case 2:
       if (!on_grouped(wdt, T, m.H)) return MX_OK;  // with qkvz in stage 1
-      return mx_project(k.dw, 1, wdt, w->ba_w, T, m.W2, m.H, h, k.v.ba, s);
+      return mx_project(k.dw, 1, wdt, T, m.W2, m.H, h, k.v.ba, s);
     case 3: {
       const dim3 grid(mx_ceil_div(m.C + m.n, 256), mx_ceil_div(T, LA_TT));
       mx_clear_error();

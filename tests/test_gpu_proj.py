@@ -120,17 +120,21 @@ def test_full_attention_projections(mi355x, stream, wdt, T):
     assert np.array_equal(out, x + y.astype(np.float32))
 
 
-@pytest.mark.parametrize("hidden,heads,dv,T", [
-    (192, 9, 256, 65),     # out: 36 stages in 4 slices, one row tile of 1 row past 64
-    (192, 9, 256, 129),    # two row tiles
-    (2048, 9, 64, 300),    # out: 9 stages, one slice; qkvz on two blocks per CU
-    (128, 8, 264, 128),    # out: 33 stages in 4 slices, the last one shorter
+@pytest.mark.parametrize("wdt,hidden,heads,dk,dv,T", [
+    ("float16", 192, 9, 32, 256, 65),    # out: 36 stages in 4 slices, one row past 64
+    ("float16", 192, 9, 32, 256, 129),   # two row tiles
+    ("float16", 2048, 9, 32, 64, 300),   # out: 9 stages, one slice; two blocks per CU
+    ("float16", 128, 8, 32, 264, 128),   # out: 33 stages in 4 slices, the last one shorter
+    ("int8", 384, 9, 32, 256, 65),       # out: 18 stages in 4 slices, the last one shorter
+    ("int8", 128, 4, 32, 1056, 129),     # out: 33 stages in 7 slices (8 would leave one empty)
+    ("int8", 128, 32, 128, 128, 1100),   # qkvz on 128 x 256 tiles, the rest on 128 x 128
+    ("int8", 256, 4, 32, 24, 70),        # out: reduction 96, on the grouped kernels
 ])
-def test_linear_attention_gemm_slices(mi355x, stream, hidden, heads, dv, T):
-    shape = syn.LinearAttnShape(hidden, heads, 32, dv, 4, 1e-6)
-    print(f"[gpu] dense GEMM hidden {hidden} vd {heads * dv} T={T}", flush=True)
+def test_linear_attention_gemm(mi355x, stream, wdt, hidden, heads, dk, dv, T):
+    shape = syn.LinearAttnShape(hidden, heads, dk, dv, 4, 1e-6)
+    print(f"[gpu] dense GEMM {wdt} hidden {hidden} vd {heads * dv} T={T}", flush=True)
     t = syn.make_linear_attn_tensors(shape, 50 + T, weight_dtype=np.float16, norm_noise=0.1)
-    w = _weights(t, (la.QKVZ, la.BA, la.OUT), "float16")
+    w = _weights(t, (la.QKVZ, la.BA, la.OUT), wdt)
     x = syn.make_inputs(51 + T, T, hidden)
     layer = DeviceLinearAttnLayer.from_host(mi355x, t, stream)
     try:
@@ -147,7 +151,7 @@ def test_linear_attention_gemm_slices(mi355x, stream, hidden, heads, dv, T):
     _check("qkvz", qkvz, h, w[la.QKVZ])
     _check("ba", ba, h, w[la.BA])
     # out = x + act W^T: one more rounding, of a sum no larger than |x| + the magnitudes
-    wo, _ = w[la.OUT]
+    wo = w[la.OUT][0] * w[la.OUT][1]
     k = act.shape[1]
     bound = ((k + 16) * 2.0 ** -24 + 2.0 ** -23) * (np.abs(act) @ np.abs(wo).T + np.abs(x)) + 1e-30
     worst = float(np.max(np.abs(out - (x + act @ wo.T)) / bound))
