@@ -63,7 +63,7 @@ struct Carve {
 struct FaWork {
   MxFullAttnViews v;
   MxDenseWork dw;  // projections: entry 0 q, 1 k, 2 v, 3 o
-  half_t* k16;     // fp16 path: keys [n_kv][Tp][DP] (Tp = T padded to 32 keys, DP = hd padded to 32)
+  half_t* k16;     // fp16 path: keys [n_kv][Tp][DP] (Tp = T padded to 64 keys, DP = padded_dim(hd))
   half_t* v16t;    // fp16 path: values per 32-key tile, transposed [n_kv][Tp / 32][DP][32]
 };
 
@@ -72,6 +72,9 @@ constexpr int FA_KT = 32;  // keys per transposed value block (fp16 path)
 #define FA_H_S32 2  // 32-key blocks per attention tile of the fp16 path
 #endif
 constexpr int FA_TPAD = FA_KT * FA_H_S32;  // keys are padded to whole tiles
+
+// Head dim of the packed fp16 keys and values: what the attention kernels are built for.
+int padded_dim(int hd) { return hd <= 32 ? 32 : hd <= 64 ? 64 : hd <= 128 ? 128 : 256; }
 
 int layout(const MxFullAttnDesc* d, int T, void* ws, FaWork* w, size_t* total) {
   MX_TRY(check_desc(d));
@@ -91,7 +94,7 @@ int layout(const MxFullAttnDesc* d, int T, void* ws, FaWork* w, size_t* total) {
   char* dwb = (char*)c.take(mx_dense_work_bytes((int)Tn, d->weight_dtype, 4));
   mx_dense_work_carve(dwb, (int)Tn, d->weight_dtype, 4, &t.dw);
   if (!f32) {
-    const size_t tp = (Tn + FA_TPAD - 1) / FA_TPAD * FA_TPAD, dp = (size_t)(m.hd + 31) / 32 * 32;
+    const size_t tp = (Tn + FA_TPAD - 1) / FA_TPAD * FA_TPAD, dp = padded_dim(m.hd);
     t.k16 = (half_t*)c.take((size_t)m.nkv * tp * dp * 2);
     t.v16t = (half_t*)c.take((size_t)m.nkv * tp * dp * 2);
   } else {
@@ -116,24 +119,188 @@ int layout(const MxFullAttnDesc* d, int T, void* ws, FaWork* w, size_t* total) {
 // per (block, frequency), not once per (token, head, dim).  Each lane recomputes its partner's
 // normalised value from memory (same rms), so there is no cross-lane exchange; all loads of
 // a row precede its reduction, all its stores follow it.
+//
+// With fp16 attention (pk.k16) the same launch writes the packed operands of the attention
+// kernels: the finished k rows go to pk.k16 as fp16 next to their fp32 form, and the first
+// n_kv_heads Tp / 32 blocks transpose one 32-key tile of a head's values through LDS (rows
+// past T and dims past head_dim are zero).  As a launch of its own the packing took 4 us at
+// one token and 19 us at 4096 (2-byte stores 64 bytes apart); RoPE and packing together went
+// 8.1 -> 3.9 us at one token, 17.5 -> 11.9 at 777, 53 -> 37 at 4096 (166 MB: 4.5 TB/s) with
+// the vector form below.
+// ------------------------------------------------------------------------------------
+__device__ __forceinline__ int fa_slot(int key) {  // key of a 32-key tile -> k-slot
+  return 8 * ((key & 15) >> 2) + (key & 3) + 4 * (key >> 4);
+}
+
+struct FaPack {
+  half_t* k16;   // keys [n_kv][Tp][DP], null for fp32 attention
+  half_t* v16t;  // values [n_kv][Tp / 32][DP][32], the keys of a tile in k-slot order
+  const float* v;
+  int Tp, DP;
+};
+
+template <int DP>
+__device__ __forceinline__ void fa_pack_values(const FaPack& pk, const FaDims& m, int T, int blk,
+                                               half_t* vt) {
+  constexpr int LD = FA_KT + 2;  // row stride in halfs: rows 4 apart start 4 banks apart
+  const int tiles = pk.Tp / FA_KT;
+  const int kvh = blk / tiles, s0 = (blk - kvh * tiles) * FA_KT;
+  constexpr int D4 = DP / 4, NP = (FA_KT * D4 + 255) / 256;
+  float4 x[NP];
+#pragma unroll
+  for (int u = 0; u < NP; ++u) {
+    const int i = threadIdx.x + 256 * u, key = i / D4, d = (i % D4) * 4, s = s0 + key;
+    x[u] = make_float4(0.f, 0.f, 0.f, 0.f);  // head_dim is a multiple of 4
+    if (key < FA_KT && s < T && d < m.hd)
+      x[u] = *(const float4*)(pk.v + (size_t)s * m.kw + (size_t)kvh * m.hd + d);
+  }
+#pragma unroll
+  for (int u = 0; u < NP; ++u) {
+    const int i = threadIdx.x + 256 * u, key = i / D4, d = (i % D4) * 4;
+    if (key >= FA_KT) break;
+    half_t* c = vt + d * LD + fa_slot(key);
+    c[0] = (half_t)x[u].x;
+    c[LD] = (half_t)x[u].y;
+    c[2 * LD] = (half_t)x[u].z;
+    c[3 * LD] = (half_t)x[u].w;
+  }
+  __syncthreads();
+  uint32_t* dst = (uint32_t*)(pk.v16t + ((size_t)kvh * pk.Tp + s0) * DP);
+#pragma unroll
+  for (int u = 0; u < DP * (FA_KT / 2) / 256; ++u) {
+    const int i = threadIdx.x + 256 * u;
+    dst[i] = *(const uint32_t*)(vt + (i / (FA_KT / 2)) * LD + 2 * (i % (FA_KT / 2)));
+  }
+  // keys past T
+  half_t* kp = pk.k16 + (size_t)kvh * pk.Tp * DP;
+  for (int i = max(s0, T) * DP + (int)threadIdx.x; i < (s0 + FA_KT) * DP; i += 256)
+    kp[i] = (half_t)0.f;
+}
+
+// The token's cos / sin table, theta^-(j / half) in fp64 and the angle rounded to fp32.
+__device__ __forceinline__ void fa_rope_table(float* cs, float* sn, int half, int t,
+                                              double theta) {
+  const int j = threadIdx.x;
+  if (j < half) {
+    const double f = 1.0 / pow(theta, (double)j / (double)half);
+    const float ang = (float)((double)t * f);
+    cs[j] = cosf(ang);
+    sn[j] = sinf(ang);
+  }
+}
+
+// The vector form, for rotary halves that are multiples of 4 dims: DP / 4 lanes per row, 4
+// dims each, 256 / DP rows per wave at once; one 16-byte load per row, partner row piece and
+// norm weight in place of four 4-byte ones, the weights loaded once per block and not once
+// per row.
+template <int DP>
+__global__ __launch_bounds__(256) void k_fa_rope_vec(float* __restrict__ qg,
+                                                     float* __restrict__ kk,
+                                                     const void* __restrict__ qn_w,
+                                                     const void* __restrict__ kn_w, int pdt,
+                                                     FaDims m, double theta, float eps,
+                                                     int rpb, FaPack pk, int T) {
+#pragma clang fp contract(off)
+  __shared__ __align__(16) float cs[128], sn[128];
+  __shared__ __align__(4) half_t vt[DP * (FA_KT + 2)];
+  const int npack = (int)gridDim.x - T;  // value tiles ahead of the tokens
+  if ((int)blockIdx.x < npack) {
+    if (blockIdx.y == 0) fa_pack_values<DP>(pk, m, T, blockIdx.x, vt);
+    return;
+  }
+  constexpr int LPR = DP / 4, RPW = 64 / LPR;
+  const int t = (int)blockIdx.x - npack, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int half = m.rd / 2;
+  fa_rope_table(cs, sn, half, t, theta);
+  const int i = 4 * (lane % LPR);
+  const bool valid = i < m.hd, rot = i < m.rd;
+  const int ic = valid ? i : 0;
+  const int p = rot ? (i < half ? i + half : i - half) : ic;  // the rotation partner's dims
+  const int jj = rot ? (i < half ? i : i - half) : 0;
+  const float4 one = make_float4(1.f, 1.f, 1.f, 1.f);
+  const float4 qw = qn_w ? mx_load_param4(qn_w, pdt, ic) : one;
+  const float4 qwp = qn_w ? mx_load_param4(qn_w, pdt, p) : one;
+  const float4 kw = kn_w ? mx_load_param4(kn_w, pdt, ic) : one;
+  const float4 kwp = kn_w ? mx_load_param4(kn_w, pdt, p) : one;
+  const int slot_end = min(m.nh + m.nkv, (int)(blockIdx.y + 1) * rpb);
+  const int first = blockIdx.y * rpb + wave * RPW;
+  auto row_of = [&](int s0) {
+    const int sl = min(s0 + lane / LPR, slot_end - 1);
+    return sl < m.nh ? qg + (size_t)t * m.qw + (size_t)sl * m.hd
+                     : kk + (size_t)t * m.kw + (size_t)(sl - m.nh) * m.hd;
+  };
+  // The first row comes in while the first wave works out the table.
+  float4 x = *(const float4*)(row_of(first) + ic), xp = *(const float4*)(row_of(first) + p);
+  __syncthreads();
+  float4 c = one, sv = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (rot) {
+    c = *(const float4*)(cs + jj);
+    sv = *(const float4*)(sn + jj);
+  }
+  if (i < half) sv = make_float4(-sv.x, -sv.y, -sv.z, -sv.w);
+  for (int s0 = first; s0 < slot_end; s0 += 4 * RPW) {
+    const bool act = s0 + lane / LPR < slot_end;
+    const int sl = min(s0 + lane / LPR, slot_end - 1);
+    const bool isq = sl < m.nh;
+    float* row = row_of(s0);
+    if (s0 != first) {
+      x = *(const float4*)(row + ic);
+      xp = *(const float4*)(row + p);
+    }
+    if (isq ? qn_w != nullptr : kn_w != nullptr) {
+      float ss = valid ? (x.x * x.x + x.y * x.y) + (x.z * x.z + x.w * x.w) : 0.f;
+      if constexpr (LPR == 64) {
+        ss = mx_wave_sum(ss);
+      } else {
+#pragma unroll
+        for (int o = 1; o < LPR; o *= 2) ss += __shfl_xor(ss, o);
+      }
+      const float rms = sqrtf(ss / (float)m.hd + eps);
+      const float4 w = isq ? qw : kw, wp = isq ? qwp : kwp;
+      x = make_float4((x.x / rms) * w.x, (x.y / rms) * w.y, (x.z / rms) * w.z, (x.w / rms) * w.w);
+      xp = make_float4((xp.x / rms) * wp.x, (xp.y / rms) * wp.y, (xp.z / rms) * wp.z,
+                       (xp.w / rms) * wp.w);
+    }
+    // y cos - y' sin (first half), y cos + y' sin (second half), y past rotary_dim
+    float4 o = x;
+    if (rot)
+      o = make_float4(x.x * c.x + xp.x * sv.x, x.y * c.y + xp.y * sv.y, x.z * c.z + xp.z * sv.z,
+                      x.w * c.w + xp.w * sv.w);
+    if (!act) continue;
+    if (valid) *(float4*)(row + i) = o;
+    if (!isq && pk.k16) {
+      typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
+      half4_t k4 = {(half_t)o.x, (half_t)o.y, (half_t)o.z, (half_t)o.w};
+      if (!valid) k4 = (half4_t){(half_t)0.f, (half_t)0.f, (half_t)0.f, (half_t)0.f};
+      *(half4_t*)(pk.k16 + ((size_t)(sl - m.nh) * pk.Tp + t) * DP + i) = k4;
+    }
+  }
+}
+
 template <int EPT>
 __global__ __launch_bounds__(256) void k_fa_rope_tok(float* __restrict__ qg,
                                                      float* __restrict__ kk,
                                                      const void* __restrict__ qn_w,
                                                      const void* __restrict__ kn_w, int pdt,
                                                      FaDims m, double theta, float eps,
-                                                     int rpb) {
+                                                     int rpb, FaPack pk, int T) {
 #pragma clang fp contract(off)
   __shared__ float cs[128], sn[128];  // rotary_dim / 2 <= head_dim / 2 <= 128
-  const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+  __shared__ __align__(4) half_t vt[64 * EPT * (FA_KT + 2)];
+  const int npack = (int)gridDim.x - T;  // value tiles ahead of the tokens
+  if ((int)blockIdx.x < npack) {
+    if (blockIdx.y > 0) return;
+    if (EPT == 1 && pk.DP == 32)
+      fa_pack_values<32>(pk, m, T, blockIdx.x, vt);
+    else
+      fa_pack_values<64 * EPT>(pk, m, T, blockIdx.x, vt);
+    return;
+  }
+  const int t = (int)blockIdx.x - npack, tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = m.rd / 2;
-  if (tid < half) {
-    const double f = 1.0 / pow(theta, (double)tid / (double)half);
-    const float ang = (float)((double)t * f);
-    cs[tid] = cosf(ang);
-    sn[tid] = sinf(ang);
-  }
+  fa_rope_table(cs, sn, half, t, theta);
   __syncthreads();
   const int slot_end = min(m.nh + m.nkv, (int)(blockIdx.y + 1) * rpb);
   for (int slot = blockIdx.y * rpb + wave; slot < slot_end; slot += 4) {
@@ -164,7 +331,12 @@ __global__ __launch_bounds__(256) void k_fa_rope_tok(float* __restrict__ qg,
 #pragma unroll
     for (int j = 0; j < EPT; ++j) {
       const int i = lane + 64 * j;
-      if (i >= m.hd) break;
+      half_t* const k16 =
+          !isq && pk.k16 ? pk.k16 + ((size_t)(slot - m.nh) * pk.Tp + t) * pk.DP : nullptr;
+      if (i >= m.hd) {
+        if (k16 && i < pk.DP) k16[i] = (half_t)0.f;
+        continue;
+      }
       const float y = nw ? (x[j] / rms) * w[j] : x[j];
       float out = y;
       if (i < m.rd) {
@@ -174,6 +346,7 @@ __global__ __launch_bounds__(256) void k_fa_rope_tok(float* __restrict__ qg,
         out = i < half ? y * c - yp * sv : y * c + yp * sv;
       }
       row[i] = out;
+      if (k16) k16[i] = (half_t)out;
     }
   }
 }
@@ -359,9 +532,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, FA_WPE))
 // output is rounded to fp16 anyway): q, k, v rounded to fp16 and both products on
 // v_mfma_f32_16x16x32_f16 with fp32 accumulation; softmax statistics stay fp32.
 //
-// k_fa_pack_kv first writes fp16 copies of the keys (after RoPE) and values: keys
-// row-major per key/value head, values transposed per 32-key tile with the keys of a
-// tile in k-slot order (below), so staging a tile is a straight 16-byte copy.
+// The RoPE launch writes fp16 copies of the keys and values: keys row-major per key/value
+// head, values transposed per 32-key tile with the keys of a tile in k-slot order (below),
+// so staging a tile is a straight 16-byte copy.
 //
 // k_fa_attn_h: block = NW waves, one query head, 16 QS NW queries (QS sets of 16 per
 // wave); tiles of 32 S32 keys, the next tile's 16-byte pieces loaded into registers while a
@@ -378,37 +551,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, FA_WPE))
 // LDS rows are padded (K: +16 B, V^T: +16 B) so the 16-byte fragment reads of a quarter
 // wave hit distinct banks.
 // ------------------------------------------------------------------------------------
-__device__ __forceinline__ int fa_slot(int key) {  // key of a 32-key tile -> k-slot
-  return 8 * ((key & 15) >> 2) + (key & 3) + 4 * (key >> 4);
-}
-
-__global__ __launch_bounds__(256) void k_fa_pack_kv(const float* __restrict__ kk,
-                                                    const float* __restrict__ vv, FaDims m,
-                                                    int T, int Tp, int DP,
-                                                    half_t* __restrict__ k16,
-                                                    half_t* __restrict__ v16t) {
-  const int nc8 = DP / 8;
-  const long i = (long)blockIdx.x * 256 + threadIdx.x;
-  const long total = (long)m.nkv * Tp * nc8;
-  if (i >= total) return;
-  const int c8 = (int)(i % nc8);
-  const long r = i / nc8;
-  const int s = (int)(r % Tp), kvh = (int)(r / Tp);
-  half8_t kh, vh;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const int d = 8 * c8 + e;
-    const bool ok = s < T && d < m.hd;
-    const size_t src = (size_t)s * m.kw + (size_t)kvh * m.hd + d;
-    kh[e] = (half_t)(ok ? kk[src] : 0.f);
-    vh[e] = (half_t)(ok ? vv[src] : 0.f);
-  }
-  *(half8_t*)(k16 + ((size_t)kvh * Tp + s) * DP + 8 * c8) = kh;
-  half_t* vt = v16t + ((size_t)kvh * (Tp / FA_KT) + s / FA_KT) * DP * FA_KT + fa_slot(s % FA_KT);
-#pragma unroll
-  for (int e = 0; e < 8; ++e) vt[(size_t)(8 * c8 + e) * FA_KT] = vh[e];
-}
-
 #ifndef FA_H_WPE
 #define FA_H_WPE 2  // waves per SIMD the fp16 attention is compiled for
 #endif
@@ -629,7 +771,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(FA_H_WP
 
 // ------------------------------------------------------------------------------------
 // k_fa_attn_d: the fp16 attention with the key / value tiles copied straight into LDS by
-// the buffer loads' LDS mode and two query sets (32 queries) per wave.
+// the buffer loads' LDS mode and QS query sets (16 queries each) per wave, two for long
+// inputs.
 // A tile is 32 keys: 2 NC key fragments (16 keys x 32 dims) and 2 NC value fragments (16
 // dims x the 32 keys in k-slot order), 1 KiB each, 32 KiB at NC = 8, double-buffered; a
 // wave's copies of tile t + 1 are issued right after the barrier that opens tile t, so
@@ -650,6 +793,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(FA_H_WP
 #endif
 #ifndef FA_D_PD
 #define FA_D_PD 2  // LDS fragment reads in flight ahead of the MFMAs
+#endif
+#ifndef FA_D_PD1
+#define FA_D_PD1 4  // the same with one query set per wave, whose registers allow more
 #endif
 #ifndef FA_D_TAU
 #define FA_D_TAU 8.f  // lazy-rescale threshold of the running max (base-2 units)
@@ -751,18 +897,22 @@ void k_fa_attn_d(const float* __restrict__ qg, const half_t* __restrict__ k16,
   const float rs = 1.4426950408889634f / sqrt_hd;
   // Queries as fp16 MFMA B fragments, four 32-dim chunks at a time (loads at clamped in-row
   // offsets, pad dims zeroed), so the staging registers stay few.
+  constexpr int QC = QS == 1 ? NC : 4;
+  // With one query set the registers hold all of a lane's query row at once, and its gate row
+  // from the start (short inputs are a chain of latencies: 24 tokens 10.8 -> 9.4 us).
+  constexpr bool GP = QS == 1;
   half8_t qf[QS][NC];
 #pragma unroll
   for (int u = 0; u < QS; ++u) {
     const float* qrow = qg + (size_t)min(qi[u], T - 1) * m.qw + (size_t)h * m.hd;
 #pragma unroll
-    for (int c0 = 0; c0 < NC; c0 += 4) {
-      float4 qv[8];
+    for (int c0 = 0; c0 < NC; c0 += QC) {
+      float4 qv[2 * QC];
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
+      for (int i = 0; i < 2 * QC; ++i)
         qv[i] = *(const float4*)(qrow + min(32 * (c0 + (i >> 1)) + 8 * g + 4 * (i & 1), m.hd - 4));
 #pragma unroll
-      for (int c = c0; c < c0 + 4 && c < NC; ++c)
+      for (int c = c0; c < c0 + QC && c < NC; ++c)
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           const float4 v = qv[2 * (c - c0) + (e >> 2)];
@@ -771,6 +921,14 @@ void k_fa_attn_d(const float* __restrict__ qg, const half_t* __restrict__ k16,
         }
       __builtin_amdgcn_sched_barrier(0);
     }
+  }
+  float4 gq[GP ? 2 * NC : 1];
+  if constexpr (GP) {
+    const float* gate = qg + (size_t)min(qi[0], T - 1) * m.qw + (size_t)m.od + (size_t)h * m.hd;
+#pragma unroll
+    for (int f = 0; f < 2 * NC; ++f)
+      gq[f] = *(const float4*)(gate + min(16 * f + 4 * g, m.hd - 4));
+    __builtin_amdgcn_sched_barrier(0);
   }
   float4_t oacc[QS][2 * NC];
 #pragma unroll
@@ -821,7 +979,7 @@ void k_fa_attn_d(const float* __restrict__ qg, const half_t* __restrict__ k16,
     auto kidx = [](int i) { return (i & 1) * NC + (i >> 1); };  // step i -> key fragment b NC + c
     // Fragment ring: step i (key steps, then the value fragments) uses fr[i % PD] and
     // refills it with step i + PD's fragment.
-    constexpr int PD = FA_D_PD;
+    constexpr int PD = QS == 1 ? FA_D_PD1 : FA_D_PD;
     auto fidx = [&](int i) { return i < NFK ? kidx(i) : i; };
     half8_t fr[PD];
 #pragma unroll
@@ -913,7 +1071,8 @@ void k_fa_attn_d(const float* __restrict__ qg, const half_t* __restrict__ k16,
       float4 gv[4];
 #pragma unroll
       for (int f = 0; f < 4; ++f)
-        gv[f] = *(const float4*)(gate + min(16 * (f0 + f) + 4 * g, m.hd - 4));
+        gv[f] = GP ? gq[GP ? f0 + f : 0]
+                   : *(const float4*)(gate + min(16 * (f0 + f) + 4 * g, m.hd - 4));
 #pragma unroll
       for (int f = 0; f < 4; ++f) {
         const int d = 16 * (f0 + f) + 4 * g;
@@ -953,16 +1112,24 @@ void k_fa_attn_d(const float* __restrict__ qg, const half_t* __restrict__ k16,
 #endif
 
 template <int NC>
-int launch_attn_h(const float* qg, const float* kk, const float* vv, const FaDims& m, int T,
-                  half_t* k16, half_t* v16t, void* act, hipStream_t s) {
-  const int Tp = (T + FA_TPAD - 1) / FA_TPAD * FA_TPAD, DP = NC * 32;
-  const long pieces = (long)m.nkv * Tp * (DP / 8);
-  mx_clear_error();
-  hipLaunchKernelGGL(k_fa_pack_kv, dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, s, kk,
-                     vv, m, T, Tp, DP, k16, v16t);
-  MX_TRY(mx_launch_status());
+int launch_attn_h(const float* qg, const FaDims& m, int T, const FaPack& pk, void* act,
+                  hipStream_t s) {
+  const half_t *k16 = pk.k16, *v16t = pk.v16t;
+  const int Tp = pk.Tp;
   const float sqrt_hd = (float)sqrt((double)m.hd);
+  mx_clear_error();
   if constexpr (FA_DMA && NC >= 4) {
+    // Two query sets per wave halve the LDS reads per product but also the blocks: they pay
+    // once those fill every CU's two block slots (16 heads: 4096 tokens 182 us against 202 with
+    // one set; 3000 tokens, 384 blocks, 140 against 116; 777 tokens 45 against 28; 24 tokens
+    // 19 against 9.4).  8-wave blocks of one set: 84 us at 2000 tokens, 2-wave ones 101,
+    // 4-wave ones 69 (two sets: 94).
+    if ((long)mx_ceil_div(T, 16 * FA_D_QS * FA_D_NW) * m.nh < 512) {
+      const dim3 grid(mx_ceil_div(T, 16 * FA_D_NW), m.nh);
+      hipLaunchKernelGGL((k_fa_attn_d<NC, FA_D_NW, 1>), grid, dim3(64 * FA_D_NW), 0, s, qg, k16,
+                         v16t, m, T, Tp, sqrt_hd, (half_t*)act);
+      return mx_launch_status();
+    }
     const dim3 grid(mx_ceil_div(T, 16 * FA_D_QS * FA_D_NW), m.nh);
     hipLaunchKernelGGL((k_fa_attn_d<NC, FA_D_NW, FA_D_QS>), grid, dim3(64 * FA_D_NW), 0, s, qg,
                        k16, v16t, m, T, Tp, sqrt_hd, (half_t*)act);
@@ -986,12 +1153,12 @@ int launch_attn(const float* qg, const float* kk, const float* vv, const FaDims&
 }
 
 int attn_launch(const float* qg, const float* kk, const float* vv, const FaDims& m, int T,
-                void* act, bool f16, half_t* k16, half_t* v16t, hipStream_t s) {
+                void* act, bool f16, const FaPack& pk, hipStream_t s) {
   if (f16) {
-    if (m.hd <= 32) return launch_attn_h<1>(qg, kk, vv, m, T, k16, v16t, act, s);
-    if (m.hd <= 64) return launch_attn_h<2>(qg, kk, vv, m, T, k16, v16t, act, s);
-    if (m.hd <= 128) return launch_attn_h<4>(qg, kk, vv, m, T, k16, v16t, act, s);
-    if (m.hd <= 256) return launch_attn_h<8>(qg, kk, vv, m, T, k16, v16t, act, s);
+    if (m.hd <= 32) return launch_attn_h<1>(qg, m, T, pk, act, s);
+    if (m.hd <= 64) return launch_attn_h<2>(qg, m, T, pk, act, s);
+    if (m.hd <= 128) return launch_attn_h<4>(qg, m, T, pk, act, s);
+    if (m.hd <= 256) return launch_attn_h<8>(qg, m, T, pk, act, s);
     return MX_ERR_UNSUPPORTED;
   }
   if (m.hd <= 16) return launch_attn<1>(qg, kk, vv, m, T, act, f16, s);
@@ -1023,6 +1190,8 @@ int run_stage(int st, const MxFullAttnDesc* d, const MxFullAttnWeights* w, const
   const int wdt = d->weight_dtype;
   const bool f32 = wdt == MX_DT_F32;
   const void* h = f32 ? (const void*)k.v.h32 : k.v.h16;
+  const FaPack pk{k.k16, k.v16t, k.v.v, (T + FA_TPAD - 1) / FA_TPAD * FA_TPAD,
+                  padded_dim(m.hd)};
   switch (st) {
     case 0:
       if (on_grouped(wdt, T, m.H) || on_grouped(wdt, T, m.od)) {
@@ -1060,24 +1229,23 @@ int run_stage(int st, const MxFullAttnDesc* d, const MxFullAttnWeights* w, const
       if (!on_grouped(wdt, T, m.H)) return MX_OK;
       return mx_project(k.dw, 2, wdt, T, m.kw, m.H, h, k.v.v, s);
     case 4: {
-      // Long inputs: one block per token (4096 tokens: 34 us against 41 us with 4 rows per
-      // block); short ones: 4 rows per block (one token: 6.8 us against 11.7 us).
-      const int rows = m.nh + m.nkv, rpb = T >= 1024 ? rows : 4;
-      const dim3 grid(T, mx_ceil_div(rows, rpb));
+      // Long inputs: one block per token (777 tokens 11.9 us against 13.4 with 4 rows per
+      // block); short ones: 4 rows per block (200 tokens: 5.3 us against 6.6).
+      const int rows = m.nh + m.nkv, rpb = T >= 512 ? rows : 4;
+      const dim3 grid(T + (f32 ? 0 : m.nkv * (pk.Tp / FA_KT)), mx_ceil_div(rows, rpb));
       mx_clear_error();
-      if (m.hd <= 64)
-        hipLaunchKernelGGL(k_fa_rope_tok<1>, grid, dim3(256), 0, s, k.v.qg, k.v.k, w->q_norm_w,
-                           w->k_norm_w, d->param_dtype, m, d->rope_theta, d->eps, rpb);
-      else if (m.hd <= 128)
-        hipLaunchKernelGGL(k_fa_rope_tok<2>, grid, dim3(256), 0, s, k.v.qg, k.v.k, w->q_norm_w,
-                           w->k_norm_w, d->param_dtype, m, d->rope_theta, d->eps, rpb);
-      else
-        hipLaunchKernelGGL(k_fa_rope_tok<4>, grid, dim3(256), 0, s, k.v.qg, k.v.k, w->q_norm_w,
-                           w->k_norm_w, d->param_dtype, m, d->rope_theta, d->eps, rpb);
+      auto* kern = m.hd <= 64 ? k_fa_rope_tok<1> : m.hd <= 128 ? k_fa_rope_tok<2> : k_fa_rope_tok<4>;
+      if (m.rd % 8 == 0)
+        kern = pk.DP == 32    ? k_fa_rope_vec<32>
+               : pk.DP == 64  ? k_fa_rope_vec<64>
+               : pk.DP == 128 ? k_fa_rope_vec<128>
+                              : k_fa_rope_vec<256>;
+      hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, k.v.qg, k.v.k, w->q_norm_w, w->k_norm_w,
+                         d->param_dtype, m, d->rope_theta, d->eps, rpb, pk, T);
       return mx_launch_status();
     }
     case 5:
-      return attn_launch(k.v.qg, k.v.k, k.v.v, m, T, k.v.act, !f32, k.k16, k.v16t, s);
+      return attn_launch(k.v.qg, k.v.k, k.v.v, m, T, k.v.act, !f32, pk, s);
     case 6:
       return mx_out_project(k.dw, 3, wdt, w->o_w, w->o_scale, T, m.H, m.od, k.v.act, k.v.y, x,
                             out, s);
