@@ -1170,8 +1170,8 @@ int attn_launch(const float* qg, const float* kk, const float* vv, const FaDims&
 }
 
 // Whether the projection with reduction length K needs the grouped kernels' tables.
-bool on_grouped(int wdt, int T, int K) {
-  return !mx_proj_ok(wdt, T, K) && !mx_dense_on_gemm(wdt, T, K);
+bool on_grouped(int wdt, int T, int K, int cols) {
+  return !mx_proj_ok(wdt, T, K) && !mx_dense_on_gemm(wdt, T, K, cols);
 }
 
 int check_weights(const MxFullAttnDesc* d, const MxFullAttnWeights* w) {
@@ -1194,7 +1194,7 @@ int run_stage(int st, const MxFullAttnDesc* d, const MxFullAttnWeights* w, const
                   padded_dim(m.hd)};
   switch (st) {
     case 0:
-      if (on_grouped(wdt, T, m.H) || on_grouped(wdt, T, m.od)) {
+      if (on_grouped(wdt, T, m.H, m.qw + 2 * m.kw) || on_grouped(wdt, T, m.od, m.H)) {
         MxDenseEntries e = {};
         e.e[0].down = w->q_w;
         e.e[0].down_scale = w->q_scale;
@@ -1209,13 +1209,13 @@ int run_stage(int st, const MxFullAttnDesc* d, const MxFullAttnWeights* w, const
       return mx_rmsnorm_launch(x, w->norm_w, d->param_dtype, d->eps, T, m.H, k.v.h32, k.v.h16,
                                s);
     case 1:
-      if (mx_proj_ok(wdt, T, m.H)) {  // q, k and v share h: one launch
+      if (mx_use_proj(wdt, T, m.H, m.qw + 2 * m.kw)) {  // q, k and v share h: one launch
         const MxProjSeg g[3] = {{w->q_w, w->q_scale, k.v.qg, m.qw, m.qw},
                                 {w->k_w, w->k_scale, k.v.k, m.kw, m.kw},
                                 {w->v_w, w->v_scale, k.v.v, m.kw, m.kw}};
         return mx_proj(wdt, h, T, m.H, g, 3, 1, s);
       }
-      if (mx_dense_on_gemm(wdt, T, m.H)) {  // q, k and v share h: one GEMM launch
+      if (mx_dense_on_gemm(wdt, T, m.H, m.qw + 2 * m.kw)) {  // q, k and v share h: one GEMM launch
         const MxGemmSeg g[3] = {{w->q_w, k.v.qg, m.qw, m.qw, nullptr, nullptr, w->q_scale},
                                 {w->k_w, k.v.k, m.kw, m.kw, nullptr, nullptr, w->k_scale},
                                 {w->v_w, k.v.v, m.kw, m.kw, nullptr, nullptr, w->v_scale}};
@@ -1223,10 +1223,10 @@ int run_stage(int st, const MxFullAttnDesc* d, const MxFullAttnWeights* w, const
       }
       return mx_project(k.dw, 0, wdt, T, m.qw, m.H, h, k.v.qg, s);
     case 2:
-      if (!on_grouped(wdt, T, m.H)) return MX_OK;  // with q in stage 1
+      if (!on_grouped(wdt, T, m.H, m.qw + 2 * m.kw)) return MX_OK;  // with q in stage 1
       return mx_project(k.dw, 1, wdt, T, m.kw, m.H, h, k.v.k, s);
     case 3:
-      if (!on_grouped(wdt, T, m.H)) return MX_OK;
+      if (!on_grouped(wdt, T, m.H, m.qw + 2 * m.kw)) return MX_OK;
       return mx_project(k.dw, 2, wdt, T, m.kw, m.H, h, k.v.v, s);
     case 4: {
       // Long inputs: one block per token (777 tokens 11.9 us against 13.4 with 4 rows per

@@ -53,10 +53,13 @@ __global__ __launch_bounds__(256) void k_residual(const float* x, float* y, long
 
 static_assert(MX_PROJ_MAX_SLICES <= MX_GEMM_MAX_SLICES, "k_residual adds either's slices");
 
+// Up to here the whole product is left in y (the header's view).
+#define MX_OUT_Y_TOKENS 64
+
 // Reduction slices of an output projection.
 int out_slices(int wdt, int T, int N, int K) {
-  if (mx_proj_ok(wdt, T, K)) return mx_proj_slices(wdt, N, K);
-  if (mx_dense_on_gemm(wdt, T, K)) return mx_gemm_slice_count(wdt, T, N, K);
+  if (mx_use_proj(wdt, T, K, N)) return mx_proj_slices(wdt, N, K);
+  if (mx_dense_on_gemm(wdt, T, K, N)) return mx_gemm_slice_count(wdt, T, N, K);
   return 1;
 }
 
@@ -77,12 +80,12 @@ int mx_out_project(const MxDenseWork& dw, int ent, int wdt, const void* w, const
                    int T, int N, int K, const void* a, float* y, const float* x, float* out,
                    hipStream_t s) {
   const int slices = out_slices(wdt, T, N, K);
-  if (mx_proj_ok(wdt, T, K)) {
+  if (mx_use_proj(wdt, T, K, N)) {
     const MxProjSeg g{w, scale, y, N, N};
     return mx_proj(wdt, a, T, K, &g, 1, slices, s);
   }
-  if (mx_dense_on_gemm(wdt, T, K)) {
-    if (slices > 1) {
+  if (mx_dense_on_gemm(wdt, T, K, N)) {
+    if (slices > 1 || T <= MX_OUT_Y_TOKENS) {
       const MxGemmSeg g{w, y, N, N, nullptr, nullptr, scale};
       return mx_gemm_slices(wdt, a, T, K, &g, slices, s);
     }
@@ -96,13 +99,14 @@ int mx_out_project(const MxDenseWork& dw, int ent, int wdt, const void* w, const
 int mx_out_residual(int wdt, int T, int N, int K, float* y, const float* x, float* out,
                     hipStream_t s) {
   const int slices = out_slices(wdt, T, N, K);
-  const bool gemm = !mx_proj_ok(wdt, T, K) && mx_dense_on_gemm(wdt, T, K);
-  if (gemm && slices == 1) return MX_OK;  // added in the GEMM's epilogue
+  const bool gemm = !mx_use_proj(wdt, T, K, N) && mx_dense_on_gemm(wdt, T, K, N);
+  if (gemm && slices == 1 && T > MX_OUT_Y_TOKENS) return MX_OK;  // added in the GEMM's epilogue
   const long n4 = (long)T * N / 4;
   const dim3 grid((unsigned)((n4 + 255) / 256));
   mx_clear_error();
   if (slices > 1)
-    hipLaunchKernelGGL(k_residual<true>, grid, dim3(256), 0, s, x, y, n4, slices, !gemm, out);
+    hipLaunchKernelGGL(k_residual<true>, grid, dim3(256), 0, s, x, y, n4, slices,
+                       T <= MX_OUT_Y_TOKENS, out);
   else
     hipLaunchKernelGGL(k_residual<false>, grid, dim3(256), 0, s, x, y, n4, 1, false, out);
   return mx_launch_status();

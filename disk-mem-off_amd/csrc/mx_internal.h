@@ -183,7 +183,9 @@ int mx_proj(int wdt, const void* a, int T, int K, const MxProjSeg* segs, int nse
 // Workspace pieces of the dense projections of an attention block (device pointers):
 // expert-table entries (one per projection), single-group m-tile tables and ones[T] for
 // the grouped-GEMM kernels, for what neither mx_proj nor mx_gemm takes.
-#define MX_DENSE_GEMM_MIN_TOKENS 65
+#define MX_DENSE_GEMM_MIN_TOKENS 33       // on mx_gemm; below, on mx_proj
+#define MX_DENSE_GEMM_MIN_TOKENS_WIDE 17  // fp16 products of at least MX_DENSE_GEMM_WIDE columns
+#define MX_DENSE_GEMM_WIDE (128 * 128)
 #define MX_DENSE_MAX_ENT 4
 struct MxDenseEntries {
   MxExpertPtrs e[MX_DENSE_MAX_ENT];  // e[i].down / down_scale = projection i's weights
@@ -200,11 +202,23 @@ size_t mx_dense_work_bytes(int T, int weight_dtype, int n_ent);
 void mx_dense_work_carve(char* base, int T, int weight_dtype, int n_ent, MxDenseWork* w);
 // Writes the table entries and m-tile tables (one small launch per block call).
 int mx_dense_setup(const MxDenseWork& w, const MxDenseEntries& ents, int T, hipStream_t s);
-// Whether projections of T tokens with these weights and reduction length K run on
-// mx_gemm (fp16 or int8 weights, long inputs, K a multiple of its stage width).
-static inline bool mx_dense_on_gemm(int wdt, int T, int K) {
-  return T >= MX_DENSE_GEMM_MIN_TOKENS && ((wdt == MX_DT_F16 && K % MX_GEMM_KMULT_F16 == 0) ||
-                                           (wdt == MX_DT_I8 && K % MX_GEMM_KMULT_I8 == 0));
+// Whether projections of T tokens onto `cols` columns (of all the segments of a launch) with
+// these weights and reduction length K run on mx_gemm: K a multiple of its stage width, and
+// enough tokens.  mx_proj re-reads the activations for every 32 columns, which overtakes the
+// GEMM's padded row tile at about 32 tokens (qkvz + ba, 20,512 columns: 32 tokens 30.4 us on
+// mx_proj, 24.8 on mx_gemm; 64 tokens 42.4 and 27.2; int8 24 tokens 19.2 and 22.2, 64 tokens
+// 32.8 and 23.9; q + k + v, 9216 columns: 32 tokens 18.9 and 20.6, 64 tokens 26.4 and 21.6), and
+// earlier where the 128-column tiles alone give the GEMM a block for every other CU.
+static inline bool mx_dense_on_gemm(int wdt, int T, int K, int cols) {
+  if (wdt == MX_DT_F16)
+    return K % MX_GEMM_KMULT_F16 == 0 &&
+           T >= (cols >= MX_DENSE_GEMM_WIDE ? MX_DENSE_GEMM_MIN_TOKENS_WIDE
+                                            : MX_DENSE_GEMM_MIN_TOKENS);
+  return wdt == MX_DT_I8 && K % MX_GEMM_KMULT_I8 == 0 && T >= MX_DENSE_GEMM_MIN_TOKENS;
+}
+// Whether they run on mx_proj.
+static inline bool mx_use_proj(int wdt, int T, int K, int cols) {
+  return mx_proj_ok(wdt, T, K) && !mx_dense_on_gemm(wdt, T, K, cols);
 }
 // y[T, N] = a[T, K] W^T with W = projection `ent`, on the grouped kernels.
 int mx_project(const MxDenseWork& w, int ent, int wdt, int T, int N, int K, const void* a,
@@ -213,7 +227,7 @@ int mx_project(const MxDenseWork& w, int ent, int wdt, int T, int N, int K, cons
 // stages: the product (into y, or straight into out where the GEMM's epilogue adds x), then
 // the residual sum (nothing to do in that case).  y holds mx_out_rows(T, N) rows of N floats:
 // the reduction slices of the product follow each other there, and the sum leaves the whole
-// product in the first T rows (not written by the GEMM forms).
+// product in the first T rows (up to 64 tokens; not written by the GEMM above).
 size_t mx_out_rows(int T, int N);
 int mx_out_project(const MxDenseWork& dw, int ent, int wdt, const void* w, const void* scale,
                    int T, int N, int K, const void* a, float* y, const float* x, float* out,

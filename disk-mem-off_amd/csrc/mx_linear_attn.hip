@@ -435,6 +435,172 @@ __global__ __launch_bounds__(256) void k_la_scan_wide(const float* __restrict__ 
   });
 }
 
+// ------------------------------------------------------------------------------------
+// Conv, gates and recurrence of short inputs in one launch (in place of k_la_prep and
+// k_la_scan_wide): the block of 16 state rows of a head forms that head's q and kb, its own
+// v rows and the decays from the projections' rows, TC tokens at a time, straight into the
+// LDS chunk the recurrence reads.  Every block of a head repeats the conv of its q and k
+// channels (dv / 16 times in all, out of L2), which costs less than the launch and the round
+// trip it replaces: a chain of one or a few tokens is latency.  The first block of a head
+// also writes the q, kb and decay rows, each block its v rows.
+// Same products and sums as k_la_prep and k_la_scan_wide, in the same order.
+// ------------------------------------------------------------------------------------
+template <int CPL, int TC, int KC>
+__global__ __launch_bounds__(256) void k_la_short(
+    const float* __restrict__ qkvz, const float* __restrict__ ba,
+    const void* __restrict__ conv_w, const void* __restrict__ a_log,
+    const void* __restrict__ dt_bias, int pdt, LaDims m, int T, int bph, float* __restrict__ q,
+    float* __restrict__ kb, float* __restrict__ v, float* __restrict__ decay,
+    float* __restrict__ o) {
+  constexpr int DK = 64 * CPL, RB = 16;
+  constexpr int NCH = (2 * DK + 255) / 256;  // q and k channels per thread
+  constexpr int NVT = (TC * RB + 255) / 256;  // v values per thread and chunk
+  __shared__ __align__(16) float sq[TC * DK], sk[TC * DK], sv[TC * RB], sd[TC];
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int h = blockIdx.x / bph;
+  const int rb0 = (blockIdx.x - h * bph) * RB;
+  const bool lead = rb0 == 0;
+  const int r0 = wave * 4, c0 = lane * CPL;
+  const int j = lane >> 4, tl = lane & 15;
+  const int row = rb0 + r0 + j;
+
+  // This thread's q / k channels: index in [q | k] of the head, column of qkvz and conv row.
+  int col[NCH];
+  bool on[NCH], isk[NCH];
+  float w[NCH][KC], win[NCH][KC];
+#pragma unroll
+  for (int u = 0; u < NCH; ++u) {
+    const int i = tid + 256 * u;
+    on[u] = i < 2 * DK;
+    isk[u] = i >= DK;
+    col[u] = on[u] ? (isk[u] ? m.qd + h * DK + i - DK : h * DK + i) : 0;
+#pragma unroll
+    for (int e = 0; e < KC; ++e) {
+      w[u][e] = mx_load_param(conv_w, pdt, col[u] * KC + e);
+      win[u][e] = 0.f;  // inputs before the first token
+    }
+  }
+  // Decay of token tid of a chunk (one wave's lanes), as in k_la_prep.
+  float ea = 0.f, bias = 0.f;
+  if (tid < TC) {
+    ea = expf(mx_load_param(a_log, pdt, h));
+    if (pdt == MX_DT_F16) ea = (float)(half_t)ea;  // np.exp of an fp16 array stays fp16
+    bias = mx_load_param(dt_bias, pdt, h);
+  }
+
+  float S[4][CPL];
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int c = 0; c < CPL; ++c) S[r][c] = 0.f;
+
+  for (int t0 = 0; t0 < T; t0 += TC) {
+    const int nt = min(TC, T - t0);
+    {
+#pragma clang fp contract(off)
+      // All of the chunk's inputs first (independent loads, tokens past T clamped).
+      float xs[NCH][TC], gs[NCH][TC], xv[NVT][KC], wv[NVT][KC], av = 0.f;
+#pragma unroll
+      for (int u = 0; u < NCH; ++u)
+#pragma unroll
+        for (int i = 0; i < TC; ++i) {
+          const size_t t = min(t0 + i, T - 1);
+          xs[u][i] = qkvz[t * m.W1 + col[u]];
+          gs[u][i] = isk[u] && on[u] ? ba[t * m.W2 + col[u] - m.qd] : 0.f;
+        }
+#pragma unroll
+      for (int u = 0; u < NVT; ++u) {
+        const int i = tid + 256 * u, t = t0 + i / RB, r = rb0 + i % RB;
+        const int c = 2 * m.qd + h * m.dv + min(r, m.dv - 1);
+#pragma unroll
+        for (int e = 0; e < KC; ++e) {
+          const int ts = min(t, T - 1) - e;
+          xv[u][e] = ts >= 0 ? qkvz[(size_t)max(ts, 0) * m.W1 + c] : 0.f;
+          wv[u][e] = mx_load_param(conv_w, pdt, c * KC + e);
+        }
+      }
+      if (tid < nt) av = ba[(size_t)(t0 + tid) * m.W2 + m.qd + h] + bias;
+      if (t0 > 0) __syncthreads();  // the previous chunk's reads are done
+#pragma unroll
+      for (int u = 0; u < NCH; ++u) {
+        float* dst = (isk[u] ? sk : sq) + ((tid + 256 * u) & (DK - 1));
+        float* g = isk[u] ? kb + col[u] - m.qd : q + col[u];
+#pragma unroll
+        for (int i = 0; i < TC; ++i) {
+#pragma unroll
+          for (int e = KC - 1; e > 0; --e) win[u][e] = win[u][e - 1];
+          win[u][0] = xs[u][i];
+          float acc = 0.f;
+#pragma unroll
+          for (int e = 0; e < KC; ++e) acc += win[u][e] * w[u][e];
+          float s = mx_silu(acc);
+          if (isk[u]) s = mx_sigmoid(gs[u][i]) * s;
+          if (on[u]) dst[i * DK] = s;
+          if (on[u] && lead && i < nt) g[(size_t)(t0 + i) * m.qd] = s;
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < NVT; ++u) {
+        const int i = tid + 256 * u, t = t0 + i / RB, r = rb0 + i % RB;
+        float acc = 0.f;
+#pragma unroll
+        for (int e = 0; e < KC; ++e) acc += xv[u][e] * wv[u][e];
+        const float s = r < m.dv ? mx_silu(acc) : 0.f;
+        if (i < TC * RB) sv[i] = s;
+        if (i < TC * RB && r < m.dv && t < T) v[(size_t)t * m.vd + h * m.dv + r] = s;
+      }
+      if (tid < nt) {
+        const float sp = av > 20.f ? av : log1pf(expf(av));
+        const float dd = expf(-ea * sp);
+        sd[tid] = dd;
+        if (lead) decay[(size_t)(t0 + tid) * m.n + h] = dd;
+      }
+    }
+    __syncthreads();
+    auto token = [&](int tt) {
+      const float4 vr = *(const float4*)(sv + tt * RB + r0);
+      const float vv[4] = {vr.x, vr.y, vr.z, vr.w};
+      const float dd = sd[tt];
+      float part[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        part[r] = 0.f;
+#pragma unroll
+        for (int c = 0; c < CPL; ++c) {
+          S[r][c] = S[r][c] * dd + vv[r] * sk[tt * DK + c0 + c];
+          part[r] += S[r][c] * sq[tt * DK + c0 + c];
+        }
+      }
+      return la_wave_sum4(part);
+    };
+    float keep = 0.f;
+    if (nt == TC) {
+#pragma unroll
+      for (int tt = 0; tt < TC; ++tt) {
+        const float ov = token(tt);
+        keep = tl == tt ? ov : keep;
+      }
+    } else {
+      for (int tt = 0; tt < nt; ++tt) {
+        const float ov = token(tt);
+        keep = tl == tt ? ov : keep;
+      }
+    }
+    if (tl < nt && row < m.dv) o[(size_t)(t0 + tl) * m.vd + h * m.dv + row] = keep;
+  }
+}
+
+// Conv kernels of 4 taps (the kernel's register window) and wide heads, up to two chunks of 16
+// tokens: one token 9.0 -> 4.7 us (conv and scan launches against this one), 24 tokens 17.5 ->
+// 15.1; at 60 tokens the repeated conv costs more than the launch (29 us).
+#define MX_LA_SHORT_T 32
+bool short_ok(const LaDims& m, int T) {
+  return T <= MX_LA_SHORT_T && m.K == 4 && (m.dk == 64 || m.dk == 128 || m.dk == 256) &&
+         (long)T * (m.W1 > m.W2 ? m.W1 : m.W2) < (1l << 31) &&
+         (long)m.n * mx_ceil_div(m.dv, 16) < (1l << 31);
+}
+
 template <int CPL, int L>
 __global__ __launch_bounds__(256) void k_la_scan(const float* __restrict__ q,
                                                  const float* __restrict__ kb,
@@ -565,8 +731,8 @@ int scan_launch(const float* q, const float* kb, const float* v, const float* de
 
 // Gated output norm: act = (w * (o / rms(o))) * silu(z) per token row (qwen3_next.py:
 // 264-266, rms_norm of _common.py:73-75), written as fp16 (fp32 for fp32 weights).
-template <int RV>
-__global__ __launch_bounds__(256) void k_la_gated_norm(const float* __restrict__ o,
+template <int RV, int NT = 256>
+__global__ __launch_bounds__(NT) void k_la_gated_norm(const float* __restrict__ o,
                                                        const float* __restrict__ qkvz,
                                                        const void* __restrict__ norm_w,
                                                        int pdt, float eps, LaDims m,
@@ -576,13 +742,13 @@ __global__ __launch_bounds__(256) void k_la_gated_norm(const float* __restrict__
   const int t = blockIdx.x;
   const float* orow = o + (size_t)t * m.vd;
   const float* z = qkvz + (size_t)t * m.W1 + 2 * m.qd + m.vd;
-  __shared__ float red[4];
+  __shared__ float red[NT / 64];
   if constexpr (RV > 0) {
-    // The row fits the register tile (vd <= 256 RV): every load is issued up front.
+    // The row fits the register tile (vd <= NT RV): every load is issued up front.
     float ov[RV], zv[RV], wv[RV];
 #pragma unroll
     for (int i = 0; i < RV; ++i) {
-      const int c = min((int)threadIdx.x + 256 * i, m.vd - 1);
+      const int c = min((int)threadIdx.x + NT * i, m.vd - 1);
       ov[i] = orow[c];
       zv[i] = z[c];
       wv[i] = mx_load_param(norm_w, pdt, c);
@@ -590,15 +756,19 @@ __global__ __launch_bounds__(256) void k_la_gated_norm(const float* __restrict__
     float ss = 0.f;
 #pragma unroll
     for (int i = 0; i < RV; ++i)
-      if ((int)threadIdx.x + 256 * i < m.vd) ss += ov[i] * ov[i];
+      if ((int)threadIdx.x + NT * i < m.vd) ss += ov[i] * ov[i];
     ss = mx_wave_sum(ss);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
     __syncthreads();
-    const float tot = (red[0] + red[1]) + (red[2] + red[3]);
+    float tot = (red[0] + red[1]) + (red[2] + red[3]);
+    if constexpr (NT > 256) {
+#pragma unroll
+      for (int i = 4; i < NT / 64; i += 4) tot += (red[i] + red[i + 1]) + (red[i + 2] + red[i + 3]);
+    }
     const float rms = sqrtf(tot / (float)m.vd + eps);
 #pragma unroll
     for (int i = 0; i < RV; ++i) {
-      const int c = threadIdx.x + 256 * i;
+      const int c = threadIdx.x + NT * i;
       if (c >= m.vd) break;
       const float a = (wv[i] * (ov[i] / rms)) * mx_silu(zv[i]);
       if (act16)
@@ -608,13 +778,13 @@ __global__ __launch_bounds__(256) void k_la_gated_norm(const float* __restrict__
     }
   } else {
     float ss = 0.f;
-    for (int c = threadIdx.x; c < m.vd; c += 256) ss += orow[c] * orow[c];
+    for (int c = threadIdx.x; c < m.vd; c += NT) ss += orow[c] * orow[c];
     ss = mx_wave_sum(ss);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
     __syncthreads();
     const float tot = (red[0] + red[1]) + (red[2] + red[3]);
     const float rms = sqrtf(tot / (float)m.vd + eps);
-    for (int c = threadIdx.x; c < m.vd; c += 256) {
+    for (int c = threadIdx.x; c < m.vd; c += NT) {
       const float a = (mx_load_param(norm_w, pdt, c) * (orow[c] / rms)) * mx_silu(z[c]);
       if (act16)
         act16[(size_t)t * m.vd + c] = (half_t)a;
@@ -625,8 +795,8 @@ __global__ __launch_bounds__(256) void k_la_gated_norm(const float* __restrict__
 }
 
 // Whether the projection with reduction length K needs the grouped kernels' tables.
-bool on_grouped(int wdt, int T, int K) {
-  return !mx_proj_ok(wdt, T, K) && !mx_dense_on_gemm(wdt, T, K);
+bool on_grouped(int wdt, int T, int K, int cols) {
+  return !mx_proj_ok(wdt, T, K) && !mx_dense_on_gemm(wdt, T, K, cols);
 }
 
 int check_weights(const MxLinearAttnDesc* d, const MxLinearAttnWeights* w) {
@@ -648,7 +818,7 @@ int run_stage(int st, const MxLinearAttnDesc* d, const MxLinearAttnWeights* w, c
   const void* h = f32 ? (const void*)k.v.h32 : k.v.h16;
   switch (st) {
     case 0:
-      if (on_grouped(wdt, T, m.H) || on_grouped(wdt, T, m.vd)) {
+      if (on_grouped(wdt, T, m.H, m.W1 + m.W2) || on_grouped(wdt, T, m.vd, m.H)) {
         MxDenseEntries e = {};
         e.e[0].down = w->qkvz_w;
         e.e[0].down_scale = w->qkvz_scale;
@@ -661,12 +831,12 @@ int run_stage(int st, const MxLinearAttnDesc* d, const MxLinearAttnWeights* w, c
       return mx_rmsnorm_launch(x, w->norm_w, d->param_dtype, d->eps, T, m.H, k.v.h32, k.v.h16,
                                s);
     case 1:
-      if (mx_proj_ok(wdt, T, m.H)) {  // qkvz and ba share h: one launch
+      if (mx_use_proj(wdt, T, m.H, m.W1 + m.W2)) {  // qkvz and ba share h: one launch
         const MxProjSeg g[2] = {{w->qkvz_w, w->qkvz_scale, k.v.qkvz, m.W1, m.W1},
                                 {w->ba_w, w->ba_scale, k.v.ba, m.W2, m.W2}};
         return mx_proj(wdt, h, T, m.H, g, 2, 1, s);
       }
-      if (mx_dense_on_gemm(wdt, T, m.H)) {  // qkvz and ba share h: one GEMM launch
+      if (mx_dense_on_gemm(wdt, T, m.H, m.W1 + m.W2)) {  // qkvz and ba share h: one GEMM launch
         const MxGemmSeg g[2] = {
             {w->qkvz_w, k.v.qkvz, m.W1, m.W1, nullptr, nullptr, w->qkvz_scale},
             {w->ba_w, k.v.ba, m.W2, m.W2, nullptr, nullptr, w->ba_scale}};
@@ -674,9 +844,10 @@ int run_stage(int st, const MxLinearAttnDesc* d, const MxLinearAttnWeights* w, c
       }
       return mx_project(k.dw, 0, wdt, T, m.W1, m.H, h, k.v.qkvz, s);
     case 2:
-      if (!on_grouped(wdt, T, m.H)) return MX_OK;  // with qkvz in stage 1
+      if (!on_grouped(wdt, T, m.H, m.W1 + m.W2)) return MX_OK;  // with qkvz in stage 1
       return mx_project(k.dw, 1, wdt, T, m.W2, m.H, h, k.v.ba, s);
     case 3: {
+      if (short_ok(m, T)) return MX_OK;  // in stage 4
       const dim3 grid(mx_ceil_div(m.C + m.n, 256), mx_ceil_div(T, LA_TT));
       mx_clear_error();
       if (m.K == 4)
@@ -690,11 +861,28 @@ int run_stage(int st, const MxLinearAttnDesc* d, const MxLinearAttnWeights* w, c
       return mx_launch_status();
     }
     case 4:
+      if (short_ok(m, T)) {
+        const int bph = mx_ceil_div(m.dv, 16);
+        // Chunks of 1, 4 or 16 tokens: a chunk's unused tokens still cost loads and conv.
+        auto* kern = m.dk == 64    ? (T == 1 ? k_la_short<1, 1, 4> : T <= 4 ? k_la_short<1, 4, 4> : k_la_short<1, 16, 4>)
+                     : m.dk == 128 ? (T == 1 ? k_la_short<2, 1, 4> : T <= 4 ? k_la_short<2, 4, 4> : k_la_short<2, 16, 4>)
+                                   : (T == 1 ? k_la_short<4, 1, 4> : T <= 4 ? k_la_short<4, 4, 4> : k_la_short<4, 16, 4>);
+        mx_clear_error();
+        hipLaunchKernelGGL(kern, dim3(m.n * bph), dim3(256), 0, s, k.v.qkvz, k.v.ba, w->conv_w,
+                           w->a_log, w->dt_bias, d->param_dtype, m, T, bph, k.v.q, k.v.kb,
+                           k.v.v, k.v.decay, k.v.o);
+        return mx_launch_status();
+      }
       return scan_launch(k.v.q, k.v.kb, k.v.v, k.v.decay, T, m.n, m.dk, m.dv, k.v.o, k.chunk_ws,
                          s);
     case 5:
       mx_clear_error();
-      if (m.vd <= 256 * 4)
+      // A row per block; few rows take 1024 threads each (one token: 4.8 -> 3.9 us).
+      if (T <= 64 && m.vd > 256 * 4 && m.vd <= 1024 * 4)
+        hipLaunchKernelGGL((k_la_gated_norm<4, 1024>), dim3(T), dim3(1024), 0, s, k.v.o, k.v.qkvz,
+                           w->out_norm_w, d->param_dtype, d->eps, m, (float*)k.v.act,
+                           f32 ? nullptr : (half_t*)k.v.act);
+      else if (m.vd <= 256 * 4)
         hipLaunchKernelGGL(k_la_gated_norm<4>, dim3(T), dim3(256), 0, s, k.v.o, k.v.qkvz,
                            w->out_norm_w, d->param_dtype, d->eps, m, (float*)k.v.act,
                            f32 ? nullptr : (half_t*)k.v.act);

@@ -363,13 +363,12 @@ typedef struct MxLinearAttnViews {
   float* y;      /* [T, H] act W_out^T; not written on the fused-GEMM path (below)      */
 } MxLinearAttnViews;
 
-/* Stages: rmsnorm, qkvz, ba, conv+gates, scan, gated norm, out, residual.  With fp16
- * (int8) weights, T >= 65 and H (for qkvz / ba) or n dv (for out) a multiple of 64 (128)
- * the projections run on the dense MFMA GEMM: ba is computed in the qkvz launch (stage 2 is
- * then empty, and the _profiled events report ba's time under qkvz), and out = x +
- * act W_out^T is formed in the out launch's epilogue (stage 7 is then empty) unless that
- * launch splits its reduction (few tokens); the view y is not written either way.  With fp16 or int8 weights and T <= 64 ba is computed in the qkvz launch
- * too.                                                                                 */
+/* Stages: rmsnorm, qkvz, ba, conv+gates, scan, gated norm, out, residual.  With fp16 or
+ * int8 weights ba is computed in the qkvz launch (stage 2 is then empty, and the _profiled
+ * events report ba's time under qkvz); short inputs form the conv and gates in the scan
+ * launch (stage 3 is then empty).  With fp16 (int8) weights, T >= 65 and n dv a multiple of
+ * 64 (128) the view y is not written: out = x + act W_out^T is formed in the out launch's
+ * epilogue (stage 7 is then empty), or from the reduction slices of that launch.        */
 #define MX_LA_N_STAGES 8
 
 int mx_linear_attn_workspace_size(const MxLinearAttnDesc* desc, int32_t tokens,
@@ -434,13 +433,12 @@ typedef struct MxFullAttnViews {
   float* y;    /* [T, H] act W_o^T; not written on the fused-GEMM path (below)          */
 } MxFullAttnViews;
 
-/* Stages: rmsnorm, q, k, v, qk-norm+rope, attention, o, residual.  With fp16 (int8)
- * weights, T >= 65 and H (for q / k / v) or n_heads head_dim (for o) a multiple of 64 (128)
- * the projections run on the dense MFMA GEMM: k and v are computed in the q launch (stages 2
- * and 3 are then empty, and the _profiled events report their time under q), and out =
- * x + act W_o^T is formed in the o launch's epilogue (stage 7 is then empty) unless that
- * launch splits its reduction (few tokens); the view y is not written either way.  With fp16 or int8 weights and T <= 64 k and v are computed in the q
- * launch too.                                                                          */
+/* Stages: rmsnorm, q, k, v, qk-norm+rope, attention, o, residual.  With fp16 or int8
+ * weights k and v are computed in the q launch (stages 2 and 3 are then empty, and the
+ * _profiled events report their time under q).  With fp16 (int8) weights, T >= 65 and
+ * n_heads head_dim a multiple of 64 (128) the view y is not written: out = x + act W_o^T is
+ * formed in the o launch's epilogue (stage 7 is then empty), or from the reduction slices of
+ * that launch.                                                                          */
 #define MX_FA_N_STAGES 8
 
 int mx_full_attn_workspace_size(const MxFullAttnDesc* desc, int32_t tokens, size_t* nbytes);
