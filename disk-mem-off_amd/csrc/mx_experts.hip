@@ -443,7 +443,8 @@ __global__ __launch_bounds__(256) void k_expert(const ExpertParams p, const Sele
 // their weights): a uniform branch per block between two copies of the tile body, no
 // spills (250-252 VGPRs).  Same box, interleaved: Qwen3-Next 4096 tokens gate/up 497 ->
 // 479 us, down 341 -> 335 us; GLM-4.7 2048-token Zipf prefill gate/up 1117 -> 1085 us,
-// down 684 -> 639 us.
+// down 684 -> 639 us.  Fragment layout only (see launch_expert_ks; GLM-4.7 rows, 200 tokens:
+// gate/up 1340 -> 1059 us, down 788 -> 635 us without the hint).
 // Block order inside an XCD run: 0 slab-major (a column slab's m-tiles in a row), 1 tile-
 // major (an m-tile's column slabs in a row), 2 expert-major (a group's blocks in a row,
 // slabs outer, its m-tiles inner: single-tile groups reuse their staged activation rows
@@ -895,7 +896,7 @@ __global__ __launch_bounds__((64 * NW), (LdsShape<WF>::OCC * 4 / NW)) void k_exp
   if constexpr (CH > 1) {
     const int items = min(CH, nslab - nb * CH);
     if ((int)threadIdx.x < trows) wrow[threadIdx.x] = p.sorted_w[p.g_start[g] + row0 + threadIdx.x];
-    if (MX_LDS_NT_SINGLE && p.g_count[g] <= MB)
+    if (MX_LDS_NT_SINGLE && p.tiled && p.g_count[g] <= MB)
       expert_lds_tile<WF, GU, 8, NBI, NW, true, CH, Y16>(p, lds, g, row0, trows, n0b, items,
                                                          wrow);
     else
@@ -905,11 +906,14 @@ __global__ __launch_bounds__((64 * NW), (LdsShape<WF>::OCC * 4 / NW)) void k_exp
   }
   if constexpr (GU && MX_LDS_HALF_TILE) {
     if (p.g_count[g] <= MB / 2) {
-      expert_lds_tile<WF, GU, 4, NBI, NW, true, 1, Y16>(p, lds, g, row0, trows, n0b);
+      if (p.tiled)
+        expert_lds_tile<WF, GU, 4, NBI, NW, true, 1, Y16>(p, lds, g, row0, trows, n0b);
+      else
+        expert_lds_tile<WF, GU, 4, NBI, NW, false, 1, Y16>(p, lds, g, row0, trows, n0b);
       return;
     }
   }
-  if (MX_LDS_NT_SINGLE && p.g_count[g] <= MB)
+  if (MX_LDS_NT_SINGLE && p.tiled && p.g_count[g] <= MB)
     expert_lds_tile<WF, GU, 8, NBI, NW, true, 1, Y16>(p, lds, g, row0, trows, n0b);
   else
     expert_lds_tile<WF, GU, 8, NBI, NW, GU ? MX_LDS_NT_GU : MX_LDS_NT_DN, 1, Y16>(
@@ -996,6 +1000,11 @@ static int decode_ksplit(bool gu, long waves_unsplit) {
   return waves_unsplit < MX_KS_DN_LO ? 4 : (waves_unsplit < MX_KS_DN_HI ? 2 : 1);
 }
 
+// The nontemporal hint goes with the fragment layout, where every load is a whole 1 KiB.  A
+// row-major load takes 64 bytes of each of 16 rows, half a 128-byte line: the line's other
+// half is the next chunk's, and with the hint it is gone by then (GLM-4.7 rows, gate/up +
+// down: one token 85.9 + 33.0 -> 60.3 + 30.3 us, 8 tokens 380 + 179 -> 288 + 161, 32 tokens
+// 999 + 445 -> 801 + 408; Qwen3-Next, 8 tokens: 61.8 + 33.1 -> 58.4 + 33.2).
 template <int WF, int MT, bool GU, int KS, int SELV = 0>
 static void launch_expert_ks(const ExpertParams& p, int mt_max, int nmax, hipStream_t s,
                              const SelectParams& sp = SelectParams{}) {
@@ -1003,9 +1012,11 @@ static void launch_expert_ks(const ExpertParams& p, int mt_max, int nmax, hipStr
   constexpr int UK = (WF == MX_DT_I8) ? (MT >= 4 ? 1 : MX_DEC_UK_I8)
                                       : (MT >= 4 ? 2 : MX_DEC_UK);
   constexpr bool NT = !(MX_I8_GU_PLAIN && WF == MX_DT_I8 && GU && MT == 1 && KS == 1);
+  auto* const kern = p.tiled ? k_expert<WF, MT, NBI, GU, UK, KS, NT, SELV>
+                             : k_expert<WF, MT, NBI, GU, UK, KS, false, SELV>;
   const dim3 grid(mt_max, mx_ceil_div(nmax, (4 / KS) * 16 * NBI));
   mx_clear_error();
-  hipLaunchKernelGGL((k_expert<WF, MT, NBI, GU, UK, KS, NT, SELV>), grid, dim3(256), 0, s, p, sp);
+  hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, p, sp);
 }
 
 template <int WF, int SELV>
