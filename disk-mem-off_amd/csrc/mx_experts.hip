@@ -843,12 +843,14 @@ static int lds_slab_chain(bool gu, int wdt, int nw, const ExpertParams& p, int m
 #ifndef MX_LDS_HALF_TILE
 #define MX_LDS_HALF_TILE 1
 #endif
-template <int WF, bool GU, int NW, int CH = 1, bool Y16 = false>
+// TILED: weights in the fragment layout; row-major ones never take the nontemporal hint.
+template <int WF, bool GU, int NW, int CH, bool Y16, bool TILED>
 __global__ __launch_bounds__((64 * NW), (LdsShape<WF>::OCC * 4 / NW)) void k_expert_lds(
     const ExpertParams p, int mt_max, int nslab) {
   constexpr int KS = 4 * WTr<WF>::EPL * LdsShape<WF>::KM;
   constexpr int NBI = GU ? 2 : 4;
   constexpr int MB = 128;
+  constexpr bool NTS = MX_LDS_NT_SINGLE && TILED;
   __shared__ __align__(16) char lds[2 * MB * (KS * 2 + MX_LDS_APAD)];
   __shared__ float wrow[CH > 1 ? MB : 1];
   const int nblk = (nslab + CH - 1) / CH;
@@ -896,7 +898,7 @@ __global__ __launch_bounds__((64 * NW), (LdsShape<WF>::OCC * 4 / NW)) void k_exp
   if constexpr (CH > 1) {
     const int items = min(CH, nslab - nb * CH);
     if ((int)threadIdx.x < trows) wrow[threadIdx.x] = p.sorted_w[p.g_start[g] + row0 + threadIdx.x];
-    if (MX_LDS_NT_SINGLE && p.tiled && p.g_count[g] <= MB)
+    if (NTS && p.g_count[g] <= MB)
       expert_lds_tile<WF, GU, 8, NBI, NW, true, CH, Y16>(p, lds, g, row0, trows, n0b, items,
                                                          wrow);
     else
@@ -906,14 +908,11 @@ __global__ __launch_bounds__((64 * NW), (LdsShape<WF>::OCC * 4 / NW)) void k_exp
   }
   if constexpr (GU && MX_LDS_HALF_TILE) {
     if (p.g_count[g] <= MB / 2) {
-      if (p.tiled)
-        expert_lds_tile<WF, GU, 4, NBI, NW, true, 1, Y16>(p, lds, g, row0, trows, n0b);
-      else
-        expert_lds_tile<WF, GU, 4, NBI, NW, false, 1, Y16>(p, lds, g, row0, trows, n0b);
+      expert_lds_tile<WF, GU, 4, NBI, NW, TILED, 1, Y16>(p, lds, g, row0, trows, n0b);
       return;
     }
   }
-  if (MX_LDS_NT_SINGLE && p.tiled && p.g_count[g] <= MB)
+  if (NTS && p.g_count[g] <= MB)
     expert_lds_tile<WF, GU, 8, NBI, NW, true, 1, Y16>(p, lds, g, row0, trows, n0b);
   else
     expert_lds_tile<WF, GU, 8, NBI, NW, GU ? MX_LDS_NT_GU : MX_LDS_NT_DN, 1, Y16>(
@@ -926,8 +925,29 @@ __global__ __launch_bounds__((64 * NW), (LdsShape<WF>::OCC * 4 / NW)) void k_exp
 #ifndef MX_PREFILL_M_BLK
 #define MX_PREFILL_M_BLK 128
 #endif
-int mx_m_blk_for(int tokens, int weight_dtype) {
+// Rows per m-tile.  A tile costs the direct-load kernel its height in activation fragment
+// loads whatever its group holds, and the 128-row kernel a barrier-paced walk; a tile too low
+// splits groups, and every tile of a group streams the group's weights (the later ones out of
+// L2).  The line is the average number of rows of a routed expert, pairs / n_experts
+// (`n_experts` 0: one group of all the rows), gate/up + down measured (MI355X, us):
+//   int8: GLM-4.7 32 tokens (1.6 rows) 311 + 171 with 16 rows, 358 + 190 with 32; 64 tokens (3.2)
+//     381 + 214 with 16, 428 + 240 with 32, 610 + 313 with 64; 100 tokens (5) 420 + 251, 468 + 274,
+//     542 + 514 with 128; Qwen3-Next 400 tokens (7.8) 218 + 117, 207 + 130, 250 + 292; GLM-4.7 400
+//     tokens (20) 952 + 541, 724 + 365, 643 + 555; 1000 tokens (50) 1464 + 775 with 32, 787 + 672
+//     with 128.
+//   fp16: Qwen3-Next 24 tokens (0.5) 126 + 66 with 16, 131 + 67 with 32; 48 tokens (0.9) 206 + 109,
+//     209 + 111, 229 + 113 with 64; 100 tokens (2) 284 + 153, 280 + 154, 286 + 168 with 128; 200
+//     tokens (3.9) 327 + 179, 313 + 179, 308 + 187; GLM-4.7 64 tokens (3.2) 739 + 406, 736 + 399,
+//     822 + 442 with 64; 200 tokens (10) 801 + 491 with 32, 780 + 482 with 128.
+int mx_m_blk_for(int tokens, int weight_dtype, long pairs, int n_experts) {
   if (tokens <= 16) return 16;
+  if (n_experts > 0 && weight_dtype == MX_DT_I8) {
+    if (pairs <= 8l * n_experts) return 16;
+    if (pairs <= 24l * n_experts) return 32;
+  } else if (n_experts > 0 && weight_dtype == MX_DT_F16) {
+    if (pairs <= n_experts) return 16;
+    if (pairs <= (tokens <= 64 ? 8l : 3l) * n_experts) return 32;
+  }
   if (tokens <= 32) return 32;
   if (tokens <= 64 || weight_dtype == MX_DT_F32) return 64;
   return MX_PREFILL_M_BLK;
@@ -1068,6 +1088,22 @@ static int dispatch_expert(int wdt, int mt, const ExpertParams& p, int mt_max, i
   return MX_ERR_INVALID;
 }
 
+template <bool GU, bool Y16, bool TILED>
+static void launch_lds_tiled(int wdt, int nw, int ch, const ExpertParams& p, int mt_max, int nblk,
+                             unsigned blocks, hipStream_t s) {
+  auto* kern = k_expert_lds<MX_DT_I8, GU, 4, 1, Y16, TILED>;
+  if (wdt == MX_DT_F16) {
+    kern = nw == 8 ? k_expert_lds<MX_DT_F16, GU, 8, 1, Y16, TILED>
+                   : k_expert_lds<MX_DT_F16, GU, 4, 1, Y16, TILED>;
+    if constexpr (!GU)
+      if (ch == 2)
+        kern = nw == 8 && MX_LDS_CHAIN8 ? k_expert_lds<MX_DT_F16, false, 8, 2, Y16, TILED>
+                                        : k_expert_lds<MX_DT_F16, false, 4, 2, Y16, TILED>;
+  }
+  mx_clear_error();
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(64 * nw), 0, s, p, mt_max, nblk);
+}
+
 // Direct-load kernel for m_blk 16/32/64; LDS-staged kernel for m_blk 128 (fp16/int8).
 // mt_max bounds the m-tile list (the kernels read the actual count from p.n_mtiles).
 template <bool GU, bool Y16>
@@ -1078,25 +1114,10 @@ static int launch_lds(int wdt, const ExpertParams& p, int mt_max, int nmax, hipS
   const int ch = lds_slab_chain(GU, wdt, nw, p, mt_max);
   const long blocks = ((long)mt_max * mx_ceil_div(nblk, ch) + 7) / 8 * 8;
   if (blocks > (1l << 31) - 1) return MX_ERR_UNSUPPORTED;
-  mx_clear_error();
-  if (!GU && ch == 2 && nw == 8 && MX_LDS_CHAIN8)
-    hipLaunchKernelGGL((k_expert_lds<MX_DT_F16, false, 8, 2, Y16>), dim3((unsigned)blocks),
-                       dim3(512), 0, s, p, mt_max, nblk);
-  else if (!GU && ch == 2)
-    hipLaunchKernelGGL((k_expert_lds<MX_DT_F16, false, 4, 2, Y16>), dim3((unsigned)blocks),
-                       dim3(256), 0, s, p, mt_max, nblk);
-  else if (!GU && ch == 4)
-    hipLaunchKernelGGL((k_expert_lds<MX_DT_F16, false, 4, 4, Y16>), dim3((unsigned)blocks),
-                       dim3(256), 0, s, p, mt_max, nblk);
-  else if (wdt == MX_DT_F16 && nw == 8)
-    hipLaunchKernelGGL((k_expert_lds<MX_DT_F16, GU, 8, 1, Y16>), dim3((unsigned)blocks),
-                       dim3(512), 0, s, p, mt_max, nblk);
-  else if (wdt == MX_DT_F16)
-    hipLaunchKernelGGL((k_expert_lds<MX_DT_F16, GU, 4, 1, Y16>), dim3((unsigned)blocks),
-                       dim3(256), 0, s, p, mt_max, nblk);
+  if (p.tiled)
+    launch_lds_tiled<GU, Y16, true>(wdt, nw, ch, p, mt_max, nblk, (unsigned)blocks, s);
   else
-    hipLaunchKernelGGL((k_expert_lds<MX_DT_I8, GU, 4, 1, Y16>), dim3((unsigned)blocks),
-                       dim3(256), 0, s, p, mt_max, nblk);
+    launch_lds_tiled<GU, Y16, false>(wdt, nw, ch, p, mt_max, nblk, (unsigned)blocks, s);
   return mx_launch_status();
 }
 

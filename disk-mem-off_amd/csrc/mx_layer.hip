@@ -80,7 +80,7 @@ int layout(const MxMoeDesc* d, int T, void* ws, MxMoeViews* v, size_t* total,
   const int S = mx_router_splits_for(Tn, d->hidden, d->n_experts, d->has_shared_gate,
                                      d->param_dtype, d->weight_dtype);
   const bool split = mx_router_on_split(Tn, d->hidden, e1, d->weight_dtype);
-  const int m_blk = mx_m_blk_for(Tn, d->weight_dtype);
+  const int m_blk = mx_m_blk_for(Tn, d->weight_dtype, (long)Tn * d->top_k, d->n_experts);
   const size_t P = (size_t)Tn * k;
   const size_t R = P + (has_sh ? Tn : 0);
   const size_t imax = d->inter > d->shared_inter ? d->inter : d->shared_inter;
