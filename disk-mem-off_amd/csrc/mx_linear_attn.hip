@@ -109,9 +109,7 @@ int layout(const MxLinearAttnDesc* d, int T, void* ws, LaWork* w, size_t* total)
 // w[c, j], summed in j order from 0 (qwen3_next.py:49-52), then silu (:238); k channels
 // times sigmoid(b) (:244, :89).  Thread C + h: g = -exp(A_log) softplus(a + dt_bias)
 // (:249), decay = exp(g) (:84).  Products are rounded before each sum, as NumPy does.
-#define LA_TT 16
-
-template <int KC>
+template <int KC, int LA_TT>
 __global__ __launch_bounds__(256) void k_la_prep(const float* __restrict__ qkvz,
                                                  const float* __restrict__ ba,
                                                  const void* __restrict__ conv_w,
@@ -436,10 +434,10 @@ __global__ __launch_bounds__(256) void k_la_scan_wide(const float* __restrict__ 
 }
 
 // ------------------------------------------------------------------------------------
-// Conv, gates and recurrence of short inputs in one launch (in place of k_la_prep and
+// Conv, gates and recurrence of at most TC tokens in one launch (in place of k_la_prep and
 // k_la_scan_wide): the block of 16 state rows of a head forms that head's q and kb, its own
-// v rows and the decays from the projections' rows, TC tokens at a time, straight into the
-// LDS chunk the recurrence reads.  Every block of a head repeats the conv of its q and k
+// v rows and the decays from the projections' rows, straight into the LDS rows the
+// recurrence reads.  Every block of a head repeats the conv of its q and k
 // channels (dv / 16 times in all, out of L2), which costs less than the launch and the round
 // trip it replaces: a chain of one or a few tokens is latency.  The first block of a head
 // also writes the q, kb and decay rows, each block its v rows.
@@ -481,7 +479,7 @@ __global__ __launch_bounds__(256) void k_la_short(
       win[u][e] = 0.f;  // inputs before the first token
     }
   }
-  // Decay of token tid of a chunk (one wave's lanes), as in k_la_prep.
+  // Decay of token tid (one wave's lanes), as in k_la_prep.
   float ea = 0.f, bias = 0.f;
   if (tid < TC) {
     ea = expf(mx_load_param(a_log, pdt, h));
@@ -495,106 +493,102 @@ __global__ __launch_bounds__(256) void k_la_short(
 #pragma unroll
     for (int c = 0; c < CPL; ++c) S[r][c] = 0.f;
 
-  for (int t0 = 0; t0 < T; t0 += TC) {
-    const int nt = min(TC, T - t0);
-    {
+  {
 #pragma clang fp contract(off)
-      // All of the chunk's inputs first (independent loads, tokens past T clamped).
-      float xs[NCH][TC], gs[NCH][TC], xv[NVT][KC], wv[NVT][KC], av = 0.f;
+    // All inputs first (independent loads, tokens past T clamped).
+    float xs[NCH][TC], gs[NCH][TC], xv[NVT][KC], wv[NVT][KC], av = 0.f;
 #pragma unroll
-      for (int u = 0; u < NCH; ++u)
+    for (int u = 0; u < NCH; ++u)
 #pragma unroll
-        for (int i = 0; i < TC; ++i) {
-          const size_t t = min(t0 + i, T - 1);
-          xs[u][i] = qkvz[t * m.W1 + col[u]];
-          gs[u][i] = isk[u] && on[u] ? ba[t * m.W2 + col[u] - m.qd] : 0.f;
-        }
-#pragma unroll
-      for (int u = 0; u < NVT; ++u) {
-        const int i = tid + 256 * u, t = t0 + i / RB, r = rb0 + i % RB;
-        const int c = 2 * m.qd + h * m.dv + min(r, m.dv - 1);
-#pragma unroll
-        for (int e = 0; e < KC; ++e) {
-          const int ts = min(t, T - 1) - e;
-          xv[u][e] = ts >= 0 ? qkvz[(size_t)max(ts, 0) * m.W1 + c] : 0.f;
-          wv[u][e] = mx_load_param(conv_w, pdt, c * KC + e);
-        }
-      }
-      if (tid < nt) av = ba[(size_t)(t0 + tid) * m.W2 + m.qd + h] + bias;
-      if (t0 > 0) __syncthreads();  // the previous chunk's reads are done
-#pragma unroll
-      for (int u = 0; u < NCH; ++u) {
-        float* dst = (isk[u] ? sk : sq) + ((tid + 256 * u) & (DK - 1));
-        float* g = isk[u] ? kb + col[u] - m.qd : q + col[u];
-#pragma unroll
-        for (int i = 0; i < TC; ++i) {
-#pragma unroll
-          for (int e = KC - 1; e > 0; --e) win[u][e] = win[u][e - 1];
-          win[u][0] = xs[u][i];
-          float acc = 0.f;
-#pragma unroll
-          for (int e = 0; e < KC; ++e) acc += win[u][e] * w[u][e];
-          float s = mx_silu(acc);
-          if (isk[u]) s = mx_sigmoid(gs[u][i]) * s;
-          if (on[u]) dst[i * DK] = s;
-          if (on[u] && lead && i < nt) g[(size_t)(t0 + i) * m.qd] = s;
-        }
+      for (int i = 0; i < TC; ++i) {
+        const size_t t = min(i, T - 1);
+        xs[u][i] = qkvz[t * m.W1 + col[u]];
+        gs[u][i] = isk[u] && on[u] ? ba[t * m.W2 + col[u] - m.qd] : 0.f;
       }
 #pragma unroll
-      for (int u = 0; u < NVT; ++u) {
-        const int i = tid + 256 * u, t = t0 + i / RB, r = rb0 + i % RB;
+    for (int u = 0; u < NVT; ++u) {
+      const int i = tid + 256 * u, t = i / RB, r = rb0 + i % RB;
+      const int c = 2 * m.qd + h * m.dv + min(r, m.dv - 1);
+#pragma unroll
+      for (int e = 0; e < KC; ++e) {
+        const int ts = min(t, T - 1) - e;
+        xv[u][e] = ts >= 0 ? qkvz[(size_t)max(ts, 0) * m.W1 + c] : 0.f;
+        wv[u][e] = mx_load_param(conv_w, pdt, c * KC + e);
+      }
+    }
+    if (tid < T) av = ba[(size_t)tid * m.W2 + m.qd + h] + bias;
+#pragma unroll
+    for (int u = 0; u < NCH; ++u) {
+      float* dst = (isk[u] ? sk : sq) + ((tid + 256 * u) & (DK - 1));
+      float* g = isk[u] ? kb + col[u] - m.qd : q + col[u];
+#pragma unroll
+      for (int i = 0; i < TC; ++i) {
+#pragma unroll
+        for (int e = KC - 1; e > 0; --e) win[u][e] = win[u][e - 1];
+        win[u][0] = xs[u][i];
         float acc = 0.f;
 #pragma unroll
-        for (int e = 0; e < KC; ++e) acc += xv[u][e] * wv[u][e];
-        const float s = r < m.dv ? mx_silu(acc) : 0.f;
-        if (i < TC * RB) sv[i] = s;
-        if (i < TC * RB && r < m.dv && t < T) v[(size_t)t * m.vd + h * m.dv + r] = s;
-      }
-      if (tid < nt) {
-        const float sp = av > 20.f ? av : log1pf(expf(av));
-        const float dd = expf(-ea * sp);
-        sd[tid] = dd;
-        if (lead) decay[(size_t)(t0 + tid) * m.n + h] = dd;
+        for (int e = 0; e < KC; ++e) acc += win[u][e] * w[u][e];
+        float s = mx_silu(acc);
+        if (isk[u]) s = mx_sigmoid(gs[u][i]) * s;
+        if (on[u]) dst[i * DK] = s;
+        if (on[u] && lead && i < T) g[(size_t)i * m.qd] = s;
       }
     }
-    __syncthreads();
-    auto token = [&](int tt) {
-      const float4 vr = *(const float4*)(sv + tt * RB + r0);
-      const float vv[4] = {vr.x, vr.y, vr.z, vr.w};
-      const float dd = sd[tt];
-      float part[4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        part[r] = 0.f;
+    for (int u = 0; u < NVT; ++u) {
+      const int i = tid + 256 * u, t = i / RB, r = rb0 + i % RB;
+      float acc = 0.f;
 #pragma unroll
-        for (int c = 0; c < CPL; ++c) {
-          S[r][c] = S[r][c] * dd + vv[r] * sk[tt * DK + c0 + c];
-          part[r] += S[r][c] * sq[tt * DK + c0 + c];
-        }
-      }
-      return la_wave_sum4(part);
-    };
-    float keep = 0.f;
-    if (nt == TC) {
-#pragma unroll
-      for (int tt = 0; tt < TC; ++tt) {
-        const float ov = token(tt);
-        keep = tl == tt ? ov : keep;
-      }
-    } else {
-      for (int tt = 0; tt < nt; ++tt) {
-        const float ov = token(tt);
-        keep = tl == tt ? ov : keep;
-      }
+      for (int e = 0; e < KC; ++e) acc += xv[u][e] * wv[u][e];
+      const float s = r < m.dv ? mx_silu(acc) : 0.f;
+      if (i < TC * RB) sv[i] = s;
+      if (i < TC * RB && r < m.dv && t < T) v[(size_t)t * m.vd + h * m.dv + r] = s;
     }
-    if (tl < nt && row < m.dv) o[(size_t)(t0 + tl) * m.vd + h * m.dv + row] = keep;
+    if (tid < T) {
+      const float sp = av > 20.f ? av : log1pf(expf(av));
+      const float dd = expf(-ea * sp);
+      sd[tid] = dd;
+      if (lead) decay[(size_t)tid * m.n + h] = dd;
+    }
   }
+  __syncthreads();
+  auto token = [&](int tt) {
+    const float4 vr = *(const float4*)(sv + tt * RB + r0);
+    const float vv[4] = {vr.x, vr.y, vr.z, vr.w};
+    const float dd = sd[tt];
+    float part[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      part[r] = 0.f;
+#pragma unroll
+      for (int c = 0; c < CPL; ++c) {
+        S[r][c] = S[r][c] * dd + vv[r] * sk[tt * DK + c0 + c];
+        part[r] += S[r][c] * sq[tt * DK + c0 + c];
+      }
+    }
+    return la_wave_sum4(part);
+  };
+  float keep = 0.f;
+  if (T == TC) {
+#pragma unroll
+    for (int tt = 0; tt < TC; ++tt) {
+      const float ov = token(tt);
+      keep = tl == tt ? ov : keep;
+    }
+  } else {
+    for (int tt = 0; tt < T; ++tt) {
+      const float ov = token(tt);
+      keep = tl == tt ? ov : keep;
+    }
+  }
+  if (tl < T && row < m.dv) o[(size_t)tl * m.vd + h * m.dv + row] = keep;
 }
 
-// Conv kernels of 4 taps (the kernel's register window) and wide heads, up to two chunks of 16
-// tokens: one token 9.0 -> 4.7 us (conv and scan launches against this one), 24 tokens 17.5 ->
-// 15.1; at 60 tokens the repeated conv costs more than the launch (29 us).
-#define MX_LA_SHORT_T 32
+// Conv kernels of 4 taps (the kernel's register window) and wide heads, up to 16 tokens: one
+// token 9.0 -> 4.7 us (conv and scan launches against this one), 6 tokens 8.0 -> 7.6, 16 tokens
+// 9.5 -> 8.9; a second chunk of 16 tokens made 24 tokens 14.9 us against 10.7.
+#define MX_LA_SHORT_T 16
 bool short_ok(const LaDims& m, int T) {
   return T <= MX_LA_SHORT_T && m.K == 4 && (m.dk == 64 || m.dk == 128 || m.dk == 256) &&
          (long)T * (m.W1 > m.W2 ? m.W1 : m.W2) < (1l << 31) &&
@@ -848,22 +842,22 @@ int run_stage(int st, const MxLinearAttnDesc* d, const MxLinearAttnWeights* w, c
       return mx_project(k.dw, 1, wdt, T, m.W2, m.H, h, k.v.ba, s);
     case 3: {
       if (short_ok(m, T)) return MX_OK;  // in stage 4
-      const dim3 grid(mx_ceil_div(m.C + m.n, 256), mx_ceil_div(T, LA_TT));
+      // Tokens per thread: few enough that short inputs fill the chip, many enough that the
+      // K - 1 re-read inputs stay few (us with 4 / 8 / 16 tokens: 48 tokens 5.4 / 6.8 / 11.4; 100
+      // 6.4 / 8.4 / 12.4; 300 12.6 / 12.0 / 16.2; 1000 30.8 / 27.3 / 30.6; 2000 61.6 / 50.6 / 51.2).
+      const int tt = T <= 160 ? 4 : T <= 1536 ? 8 : 16;
+      const dim3 grid(mx_ceil_div(m.C + m.n, 256), mx_ceil_div(T, tt));
+      auto* kern = m.K == 4 ? (tt == 4 ? k_la_prep<4, 4> : tt == 8 ? k_la_prep<4, 8> : k_la_prep<4, 16>)
+                            : (tt == 4 ? k_la_prep<0, 4> : tt == 8 ? k_la_prep<0, 8> : k_la_prep<0, 16>);
       mx_clear_error();
-      if (m.K == 4)
-        hipLaunchKernelGGL(k_la_prep<4>, grid, dim3(256), 0, s, k.v.qkvz, k.v.ba, w->conv_w,
-                           w->a_log, w->dt_bias, d->param_dtype, m, T, k.v.q, k.v.kb, k.v.v,
-                           k.v.decay);
-      else
-        hipLaunchKernelGGL(k_la_prep<0>, grid, dim3(256), 0, s, k.v.qkvz, k.v.ba, w->conv_w,
-                           w->a_log, w->dt_bias, d->param_dtype, m, T, k.v.q, k.v.kb, k.v.v,
-                           k.v.decay);
+      hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, k.v.qkvz, k.v.ba, w->conv_w, w->a_log,
+                         w->dt_bias, d->param_dtype, m, T, k.v.q, k.v.kb, k.v.v, k.v.decay);
       return mx_launch_status();
     }
     case 4:
       if (short_ok(m, T)) {
         const int bph = mx_ceil_div(m.dv, 16);
-        // Chunks of 1, 4 or 16 tokens: a chunk's unused tokens still cost loads and conv.
+        // Built for 1, 4 and 16 tokens: unused tokens still cost loads and conv.
         auto* kern = m.dk == 64    ? (T == 1 ? k_la_short<1, 1, 4> : T <= 4 ? k_la_short<1, 4, 4> : k_la_short<1, 16, 4>)
                      : m.dk == 128 ? (T == 1 ? k_la_short<2, 1, 4> : T <= 4 ? k_la_short<2, 4, 4> : k_la_short<2, 16, 4>)
                                    : (T == 1 ? k_la_short<4, 1, 4> : T <= 4 ? k_la_short<4, 4, 4> : k_la_short<4, 16, 4>);
