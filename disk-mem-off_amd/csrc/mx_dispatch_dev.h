@@ -72,6 +72,49 @@ __device__ __forceinline__ void mx_dispatch_scan(const int* tot, int* off, int* 
   }
 }
 
+// The same scans for small batches (T k <= 2048) with one expert per thread (E <= blockDim.x):
+// rows and tiles packed into the halves of one word, so a wave takes one shuffle scan and a
+// ballot, and the waves' totals (at most 16) are added across.  Wave 0 alone walked E / 64
+// experts per lane, with a division by m_blk at each, while 15 waves waited.
+__device__ __forceinline__ void mx_dispatch_scan_wide(int n, int* off, int* gid, int* mtb,
+                                                      int* s_tot, int E, int m_blk) {
+  __shared__ uint32_t wsum[16], wact[16];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, nw = blockDim.x >> 6;
+  if (tid >= E) n = 0;
+  const uint32_t v = (uint32_t)n | (uint32_t)((n + m_blk - 1) / m_blk) << 16;
+  uint32_t inc = v;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const uint32_t x = __shfl_up(inc, d, 64);
+    if (lane >= d) inc += x;
+  }
+  const unsigned long long act = __ballot(n > 0);
+  if (lane == 63) {
+    wsum[w] = inc;
+    wact[w] = __popcll(act);
+  }
+  mx_lds_sync();
+  uint32_t base = 0, abase = 0, total = 0, atotal = 0;
+  for (int i = 0; i < nw; ++i) {
+    const uint32_t s = wsum[i], a = wact[i];
+    base += i < w ? s : 0;
+    abase += i < w ? a : 0;
+    total += s;
+    atotal += a;
+  }
+  const uint32_t ex = base + inc - v;
+  if (tid < E) {
+    off[tid] = ex & 0xffff;
+    mtb[tid] = ex >> 16;
+    gid[tid] = abase + __popcll(act & ((1ull << lane) - 1ull));
+  }
+  if (tid == 0) {
+    s_tot[0] = total & 0xffff;
+    s_tot[1] = atotal;
+    s_tot[2] = total >> 16;
+  }
+}
+
 // Offsets, group table, m-tile list and the shared-expert rows, from the scanned tables.
 __device__ __forceinline__ void mx_dispatch_tail(
     const int* tot, const int* off, const int* gid, const int* mtb, const int* s_tot, int T,
@@ -244,13 +287,22 @@ __device__ __forceinline__ void mx_dispatch_block_small(
     if ((unsigned)e < (unsigned)E) atomicOr(&mask[e], 1ull << (p / k));
   }
   mx_lds_sync();
-  for (int e = tid; e < E; e += nt) {
-    const int n = __popcll(mask[e]);
-    tot[e] = n;
-    counts[e] = n;
+  if (E <= nt) {
+    const int n = tid < E ? __popcll(mask[tid]) : 0;
+    if (tid < E) {
+      tot[tid] = n;
+      counts[tid] = n;
+    }
+    mx_dispatch_scan_wide(n, off, gid, mtb, s_tot, E, m_blk);
+  } else {
+    for (int e = tid; e < E; e += nt) {
+      const int n = __popcll(mask[e]);
+      tot[e] = n;
+      counts[e] = n;
+    }
+    mx_lds_sync();
+    mx_dispatch_scan(tot, off, gid, mtb, s_tot, E, m_blk);
   }
-  mx_lds_sync();
-  mx_dispatch_scan(tot, off, gid, mtb, s_tot, E, m_blk);
   mx_lds_sync();
   for (int p = tid; p < P; p += nt) {
     const int e = ids[p], t = p / k;

@@ -560,15 +560,16 @@ extern "C" int mx_router_topk(const float* logits, int32_t splits, const void* b
 }
 
 // ------------------------------------------------------------------------------------
-// Decode router (T <= 64): two launches, the RMSNorm folded into the first.
-//   k_router_logits_decode: one block per (expert row, group of up to 8 tokens) over the
-//     full H (no H split); also writes the normalised activations.
+// Decode router (T <= 64): two or three launches, the RMSNorm folded into the first.
+//   k_router_logits_decode: one block per (1, 2 or 4 expert rows, group of up to 8 tokens)
+//     over the full H (no H split); also writes the normalised activations.
 //   k_topk_dispatch: one workgroup of up to 16 waves; per-token top-k (one wave per
-//     token), then the dispatch.  A kernel boundary separates the two: the blocks of the
+//     token), then the dispatch.  More tokens than its waves: k_router_topk and
+//     k_dispatch_few, a third launch.  A kernel boundary separates the two: the blocks of the
 //     logits kernel run on every XCD, and publishing their results inside one launch
 //     would need an L2 write-back per block.
 // ------------------------------------------------------------------------------------
-// Block (e, g): expert row e (row E = Qwen3-Next shared gate) against tokens g*TT ..
+// Block (b, g): expert rows b*EB .. (row E = Qwen3-Next shared gate) against tokens g*TT ..
 // g*TT+TT-1, with the RMSNorm folded in: each lane accumulates x . (norm_w * w_e) and
 // x . x over its H columns, the 4 waves (H quarters) are added in LDS in a fixed order,
 // and logit = dot / rms with rms = sqrt(mean(x^2) + eps) (_common.py:73-75).  The blocks
@@ -578,71 +579,86 @@ extern "C" int mx_router_topk(const float* logits, int32_t splits, const void* b
 // At most 2 waves per SIMD: the register budget lets every load of a loop step be
 // issued before the first FMA waits (at the default occupancy target the compiler
 // serialises load -> wait -> FMA per token row).
-template <typename WT, int TT>
+template <typename WT, int TT, int EB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void
 k_router_logits_decode(
     const float* __restrict__ x, const WT* __restrict__ norm_w, float eps,
     const WT* __restrict__ wr, const WT* __restrict__ wseg, int T, int H, int E, int E1,
     float* __restrict__ logits, float* __restrict__ h32, half_t* __restrict__ h16) {
-  __shared__ float part[4][TT], sq[4][TT];
+  __shared__ float part[4][EB][TT], sq[4][TT];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int e = blockIdx.x;
+  const int e0 = blockIdx.x * EB;
   const int t0 = blockIdx.y * TT;
-  const WT* row = (e < E) ? wr + (size_t)e * H : wseg;
+  const WT* row[EB];
+#pragma unroll
+  for (int b = 0; b < EB; ++b) {
+    const int e = min(e0 + b, E1 - 1);
+    row[b] = e < E ? wr + (size_t)e * H : wseg;
+  }
   // One sweep of the wave covers 64 lanes x 4 columns; the loop stride is that sweep and
   // does not follow the prefill router's slice width.
   constexpr int SWEEP = 64 * 4;
   const int hq = (H / 4 + SWEEP - 1) / SWEEP * SWEEP;  // H quarter per wave, whole sweeps
   const int kb = wave * hq, ke = min(H, kb + hq);
-  float acc[TT], ss[TT];
+  float acc[EB][TT], ss[TT];
   const float* xrow[TT];
 #pragma unroll
   for (int t = 0; t < TT; ++t) {
-    acc[t] = 0.f;
+#pragma unroll
+    for (int b = 0; b < EB; ++b) acc[b][t] = 0.f;
     ss[t] = 0.f;
     xrow[t] = x + (size_t)min(t0 + t, T - 1) * H;
   }
 #pragma unroll 4
   for (int c = kb + lane * 4; c < ke; c += SWEEP) {
-    const float4 wv = rt_load4<WT>(row + c);
+    float4 g[EB];
     const float4 nv = rt_load4<WT>(norm_w + c);
-    const float4 g = make_float4(nv.x * wv.x, nv.y * wv.y, nv.z * wv.z, nv.w * wv.w);
+#pragma unroll
+    for (int b = 0; b < EB; ++b) {
+      const float4 wv = rt_load4<WT>(row[b] + c);
+      g[b] = make_float4(nv.x * wv.x, nv.y * wv.y, nv.z * wv.z, nv.w * wv.w);
+    }
 #pragma unroll
     for (int t = 0; t < TT; ++t) {
       const float4 xv = *(const float4*)(xrow[t] + c);
-      float a = acc[t], q = ss[t];
-      a = fmaf(xv.x, g.x, a);
+      float q = ss[t];
       q = fmaf(xv.x, xv.x, q);
-      a = fmaf(xv.y, g.y, a);
       q = fmaf(xv.y, xv.y, q);
-      a = fmaf(xv.z, g.z, a);
       q = fmaf(xv.z, xv.z, q);
-      a = fmaf(xv.w, g.w, a);
-      q = fmaf(xv.w, xv.w, q);
-      acc[t] = a;
-      ss[t] = q;
+      ss[t] = fmaf(xv.w, xv.w, q);
+#pragma unroll
+      for (int b = 0; b < EB; ++b) {
+        float a = acc[b][t];
+        a = fmaf(xv.x, g[b].x, a);
+        a = fmaf(xv.y, g[b].y, a);
+        a = fmaf(xv.z, g[b].z, a);
+        acc[b][t] = fmaf(xv.w, g[b].w, a);
+      }
     }
   }
 #pragma unroll
   for (int t = 0; t < TT; ++t) {
-    const float v = mx_wave_sum(acc[t]);
     const float q = mx_wave_sum(ss[t]);
-    if (lane == 0) {
-      part[wave][t] = v;
-      sq[wave][t] = q;
+    if (lane == 0) sq[wave][t] = q;
+#pragma unroll
+    for (int b = 0; b < EB; ++b) {
+      const float v = mx_wave_sum(acc[b][t]);
+      if (lane == 0) part[wave][b][t] = v;
     }
   }
   __syncthreads();
-  if (threadIdx.x < TT && t0 + (int)threadIdx.x < T) {
-    const int t = threadIdx.x;
+  const int bt = threadIdx.x / TT;
+  if (bt < EB && e0 + bt < E1 && t0 + (int)threadIdx.x % TT < T) {
+    const int t = threadIdx.x % TT;
     const float rms = sqrtf(((sq[0][t] + sq[1][t]) + (sq[2][t] + sq[3][t])) / (float)H + eps);
-    logits[(size_t)(t0 + t) * E1 + e] = ((part[0][t] + part[1][t]) + (part[2][t] + part[3][t])) / rms;
+    logits[(size_t)(t0 + t) * E1 + e0 + bt] =
+        ((part[0][bt][t] + part[1][bt][t]) + (part[2][bt][t] + part[3][bt][t])) / rms;
   }
   // Normalised rows of this token group, spread over all blocks of the group: one
   // float4 per thread (the x reads hit L2).  Every block reduced the same values in the
   // same order, so all of them hold the same rms.
   const int ng = min(TT, T - t0), h4 = H / 4;
-  for (int i = e * 256 + (int)threadIdx.x; i < ng * h4; i += E1 * 256) {
+  for (int i = blockIdx.x * 256 + (int)threadIdx.x; i < ng * h4; i += (int)gridDim.x * 256) {
     const int t = i / h4, c = (i - t * h4) * 4;
     const float rms = sqrtf(((sq[0][t] + sq[1][t]) + (sq[2][t] + sq[3][t])) / (float)H + eps);
     const size_t o = (size_t)(t0 + t) * H + c;
@@ -709,6 +725,20 @@ __global__ __launch_bounds__(VPT > 8 ? 512 : 1024) void k_topk_dispatch(
                           g_count, n_groups, mt_group, mt_row0, n_mtiles);
 }
 
+// The dispatch part alone, of tokens selected by k_router_topk.
+__global__ __launch_bounds__(1024) void k_dispatch_few(
+    const int* __restrict__ ids, const float* __restrict__ tw, const float* __restrict__ shared_w,
+    int T, int E, int k, int has_shared, int m_blk, int* __restrict__ counts,
+    int* __restrict__ offsets, int* __restrict__ sorted_tok, float* __restrict__ sorted_w,
+    int* __restrict__ pair_pos, int* __restrict__ g_expert, int* __restrict__ g_start,
+    int* __restrict__ g_count, int* __restrict__ n_groups, int* __restrict__ mt_group,
+    int* __restrict__ mt_row0, int* __restrict__ n_mtiles) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  mx_dispatch_block_small(smem, ids, tw, shared_w, T, k, E, has_shared, m_blk, counts, offsets,
+                          sorted_tok, sorted_w, pair_pos, g_expert, g_start, g_count, n_groups,
+                          mt_group, mt_row0, n_mtiles);
+}
+
 // Dynamic LDS of the top-k/dispatch workgroup: dispatch tables, then the staged top-k
 // results (the top-k rows and the small-batch candidates take about 15 KB of static LDS
 // besides, so 48 KB of dynamic LDS keeps the workgroup within 64 KB).
@@ -745,15 +775,25 @@ int mx_router_decode_launch(const MxMoeDesc* d, const MxMoeWeights* w, int T, co
   const void* b = (d->router_mode == MX_ROUTER_SOFTMAX || !d->has_bias) ? nullptr : w->bias;
   const void* seg = d->has_shared_gate ? w->shared_gate_w : nullptr;
   mx_clear_error();
-#define RL_LAUNCH(WT_, TT_)                                                                    \
-  hipLaunchKernelGGL((k_router_logits_decode<WT_, TT_>), dim3(e1, mx_ceil_div(T, TT_)),        \
-                     dim3(256), 0, s, x, (const WT_*)w->norm_w, d->eps, (const WT_*)w->router_w, \
+  // Expert rows per block, from the blocks that one row each would make: 2 once they are past
+  // the 512 the chip holds at 2 waves per SIMD, 4 past twice that; below, fewer blocks lose
+  // more than the shared x loads give (GLM-4.7 shape, 8 tokens, 160 blocks: 6.6 us with one
+  // row, 7.7 with two; 16 tokens 8.0 / 8.4).  One / two / four rows in us: Qwen3-Next shape 8
+  // tokens 7.4 / 6.0 / -, 24 tokens 14.0 / 10.6 / 8.8, 64 tokens 31.9 / 23.8 / 20.4; GLM-4.7
+  // shape 32 tokens 11.7 / 10.0 / -, 64 tokens 17.6 / 14.6 / 12.8.
+  const int blocks8 = e1 * mx_ceil_div(T, 8);
+#define RL_LAUNCH(WT_, TT_, EB_)                                                               \
+  hipLaunchKernelGGL((k_router_logits_decode<WT_, TT_, EB_>),                                  \
+                     dim3(mx_ceil_div(e1, EB_), mx_ceil_div(T, TT_)), dim3(256), 0, s, x,      \
+                     (const WT_*)w->norm_w, d->eps, (const WT_*)w->router_w,                  \
                      (const WT_*)seg, T, H, E, e1, logits, h32, (half_t*)h16)
 #define RL_TT(WT_)                                  \
-  if (T <= 1) RL_LAUNCH(WT_, 1);                    \
-  else if (T <= 2) RL_LAUNCH(WT_, 2);               \
-  else if (T <= 4) RL_LAUNCH(WT_, 4);               \
-  else RL_LAUNCH(WT_, 8);
+  if (T <= 1) RL_LAUNCH(WT_, 1, 1);                 \
+  else if (T <= 2) RL_LAUNCH(WT_, 2, 1);            \
+  else if (T <= 4) RL_LAUNCH(WT_, 4, 1);            \
+  else if (blocks8 <= 512) RL_LAUNCH(WT_, 8, 1);    \
+  else if (blocks8 <= 1024) RL_LAUNCH(WT_, 8, 2);   \
+  else RL_LAUNCH(WT_, 8, 4);
   if (d->param_dtype == MX_DT_F16) {
     RL_TT(half_t)
   } else {
@@ -763,6 +803,20 @@ int mx_router_decode_launch(const MxMoeDesc* d, const MxMoeWeights* w, int T, co
 #undef RL_LAUNCH
   MX_TRY(mx_launch_status());
   if (select_later) return MX_OK;
+  // Past one token per wave the one workgroup selects in rounds, four waves to a SIMD; a wave per
+  // token over the chip and the dispatch in a launch of its own are shorter (us, one launch /
+  // two): 512 experts 16 tokens 13.0 / 12.1, 24 tokens 16.9 / 12.1, 64 tokens 36.2 / 12.9; 160
+  // experts 16 tokens 9.7 / 10.5, 32 tokens 13.8 / 10.3, 64 tokens 22.0 / 10.6.
+  if (T > nw && d->top_k <= E) {
+    MX_TRY(mx_router_topk(logits, 1, b, d->param_dtype, T, E, d->top_k, d->router_mode,
+                          d->norm_topk_prob, d->routed_scaling, d->has_shared_gate, ids, tw,
+                          shared_w, s));
+    hipLaunchKernelGGL(k_dispatch_few, dim3(1), dim3(1024), mx_dispatch_small_lds_bytes(E), s,
+                       ids, tw, shared_w, T, E, d->top_k, has_shared, m_blk, counts, offsets,
+                       sorted_tok, sorted_w, pair_pos, g_expert, g_start, g_count, n_groups,
+                       mt_group, mt_row0, n_mtiles);
+    return mx_launch_status();
+  }
   // One token with a single-wave selection needs one wave only.
   const int nwl = (T == 1 && vpt < 6) ? 1 : nw;
 #define TD_LAUNCH(V)                                                                           \
