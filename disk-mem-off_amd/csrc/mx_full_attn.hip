@@ -189,7 +189,8 @@ __device__ __forceinline__ void fa_rope_table(float* cs, float* sn, int half, in
   }
 }
 
-// The vector form, for rotary halves that are multiples of 4 dims: DP / 4 lanes per row, 4
+// The vector form, for rotary halves that are multiples of 4 dims and norm weights on a
+// 16-byte boundary (the scalar form takes them at any address): DP / 4 lanes per row, 4
 // dims each, 256 / DP rows per wave at once; one 16-byte load per row, partner row piece and
 // norm weight in place of four 4-byte ones, the weights loaded once per block and not once
 // per row.
@@ -1235,7 +1236,7 @@ int run_stage(int st, const MxFullAttnDesc* d, const MxFullAttnWeights* w, const
       const dim3 grid(T + (f32 ? 0 : m.nkv * (pk.Tp / FA_KT)), mx_ceil_div(rows, rpb));
       mx_clear_error();
       auto* kern = m.hd <= 64 ? k_fa_rope_tok<1> : m.hd <= 128 ? k_fa_rope_tok<2> : k_fa_rope_tok<4>;
-      if (m.rd % 8 == 0)
+      if (m.rd % 8 == 0 && mx_aligned16(w->q_norm_w) && mx_aligned16(w->k_norm_w))
         kern = pk.DP == 32    ? k_fa_rope_vec<32>
                : pk.DP == 64  ? k_fa_rope_vec<64>
                : pk.DP == 128 ? k_fa_rope_vec<128>

@@ -66,3 +66,30 @@ def test_attention_matches_oracle(mi355x, stream, hd, nh, nkv, T):
     err = np.linalg.norm(act - want) / np.linalg.norm(want)
     print(f"    normwise err {err:.2e}", flush=True)
     assert np.all(np.isfinite(act)) and err <= 4 * 2.0 ** -11
+
+
+def test_norm_weights_at_any_address(mi355x, stream):
+    """q / k norm weights off the 16-byte boundary take the scalar RoPE form: same block output
+    up to the order of the row sums (fp32) and the fp16 roundings after them."""
+    hd, nh, nkv, T = 64, 4, 2, 37
+    print(f"[gpu] norm weights 4 bytes off, hd={hd} T={T}", flush=True)
+    s = syn.FullAttnShape(128, nh, nkv, hd, 0.25, 10000.0, 1e-6)
+    t = syn.make_full_attn_tensors(s, 7, weight_dtype=np.float16, norm_noise=0.1)
+    x = syn.make_inputs(8, T, s.hidden)
+    layer = DeviceFullAttnLayer.from_host(mi355x, t, nh, nkv, hd, s.rotary_dim, s.rope_theta,
+                                          stream)
+    raw = np.concatenate([np.zeros(1), t["self_attn.q_norm.weight"].ravel(),
+                          t["self_attn.k_norm.weight"].ravel()]).astype(np.float32)
+    buf = mi355x.alloc_device(raw.nbytes)
+    try:
+        want = layer.forward_numpy(x, s.eps)
+        mi355x.copy_h2d_ptr_async(buf.handle, raw.ctypes.data, raw.nbytes, stream)
+        mi355x.synchronize_stream(stream)
+        w = layer.weights()
+        w.q_norm_w = int(buf.handle) + 4
+        w.k_norm_w = int(buf.handle) + 4 + 4 * hd
+        got = layer.runner.forward_numpy(layer.desc(s.eps), w, x, stream)
+    finally:
+        mi355x.free_device(buf)
+        layer.close()
+    assert np.linalg.norm(got - want) <= 4 * 2.0 ** -11 * np.linalg.norm(want - x)
