@@ -125,6 +125,37 @@ int layout(const MxMoeDesc* d, int T, void* ws, MxMoeViews* v, size_t* total,
   return MX_OK;
 }
 
+// What a workspace needs to serve `T` tokens and every shorter input.  layout() alone can
+// fall as T grows: the router cuts its reduction into fewer slices once the rows fill the
+// chip (Qwen3-Next shape: 512 tokens take 5 MB more than 513), and higher m-tiles make
+// shorter lists.  Between two changes of those it only rises, so its value right before each
+// change and at T itself bound the rest.
+int workspace_bound(const MxMoeDesc* d, int T, size_t* total) {
+  MX_TRY(layout(d, T, nullptr, nullptr, total));
+  const int e1 = d->n_experts + (d->has_shared_gate ? 1 : 0);
+  struct Key {
+    int splits, m_blk;
+    bool split_planes;
+  };
+  auto key = [&](int t) {
+    return Key{mx_router_splits_for(t, d->hidden, d->n_experts, d->has_shared_gate,
+                                    d->param_dtype, d->weight_dtype),
+               mx_m_blk_for(t, d->weight_dtype, (long)t * d->top_k, d->n_experts),
+               mx_router_on_split(t, d->hidden, e1, d->weight_dtype)};
+  };
+  Key next = key(T > 0 ? T : 1);
+  for (int t = T - 1; t >= 1; --t) {
+    const Key k = key(t);
+    if (k.splits != next.splits || k.m_blk != next.m_blk || k.split_planes != next.split_planes) {
+      size_t n = 0;
+      MX_TRY(layout(d, t, nullptr, nullptr, &n));
+      if (n > *total) *total = n;
+    }
+    next = k;
+  }
+  return MX_OK;
+}
+
 // One token, when stages 1-4 run in one call: the gate/up launch selects the experts
 // (and writes the dispatch tables), so the top-k/dispatch launch is left out.
 #ifndef MX_SELECT_IN_GATE_UP
@@ -262,7 +293,7 @@ int forward(const MxMoeDesc* d, const MxMoeWeights* w, const float* x, float* ou
 
 extern "C" int mx_moe_workspace_size(const MxMoeDesc* desc, int32_t tokens, size_t* nbytes) {
   if (!nbytes) return MX_ERR_INVALID;
-  return layout(desc, tokens, nullptr, nullptr, nbytes);
+  return workspace_bound(desc, tokens, nbytes);
 }
 
 extern "C" int mx_moe_views(const MxMoeDesc* desc, int32_t tokens, void* workspace,

@@ -184,6 +184,8 @@ int mx_event_elapsed_ms(float* ms, void* start, void* end);    /* no counterpart
  *   out = x + sum_j w[t,j] * SwiGLU_{id[t,j]}(h[t]) + shared_w[t] * SwiGLU_shared(h[t]) *
  *   with h = rms_norm(x).  x and out are fp32 [T, H] device buffers (may not alias).    *
  * =================================================================================== */
+/* Bytes of workspace that serve `tokens` tokens and every shorter input; never less for
+ * more tokens.                                                                        */
 int mx_moe_workspace_size(const MxMoeDesc* desc, int32_t tokens, size_t* nbytes);
 int mx_moe_views(const MxMoeDesc* desc, int32_t tokens, void* workspace, MxMoeViews* views);
 int mx_moe_forward(const MxMoeDesc* desc, const MxMoeWeights* weights, const float* x,
@@ -213,7 +215,8 @@ int mx_moe_forward_profiled(const MxMoeDesc* desc, const MxMoeWeights* weights,
  * hipMalloc.  The same computation, without the workspace arguments: the stages run out of
  * a scratch array of MX_NOALLOC_MAX_WORKSPACE bytes that the library holds on every device
  * it runs on until the process ends.  Nothing is allocated and no memset is issued.
- * Returns MX_ERR_WORKSPACE when mx_moe_workspace_size(desc, tokens) exceeds that size;
+ * Returns MX_ERR_WORKSPACE when the call's own buffers exceed that size, never when
+ * mx_moe_workspace_size(desc, tokens) does not;
  * size batches from that function, not from the token count alone (from 65 tokens the
  * prefill-path buffers join the workspace).  With 16 MiB: GLM-4.7 shapes up to 64 tokens
  * (62 with fp32 experts), Qwen3-Next shapes up to 83 (108 with fp32 experts).  Every call on

@@ -54,6 +54,20 @@ def test_workspace_size_grows_with_tokens():
     assert rc1 == rc2 == _lib.MX_OK and 0 < n1 < n2
 
 
+@pytest.mark.parametrize("wdt", [_lib.MX_DT_F32, _lib.MX_DT_F16, _lib.MX_DT_I8])
+@pytest.mark.parametrize("shape", [
+    dict(hidden=5120, inter=1536, shared_inter=1536, n_experts=160, top_k=8),
+    dict(hidden=2048, inter=512, shared_inter=512, n_experts=512, top_k=10, has_bias=0,
+         has_shared_gate=1),
+    dict(hidden=64, inter=32, shared_inter=0, n_experts=1024, top_k=1)])
+def test_moe_workspace_never_shrinks_with_tokens(wdt, shape):
+    """A workspace sized for a batch serves every shorter one (the runners size it once), although
+    the router's slices and the m-tile lists get fewer as tokens grow."""
+    d = _desc(weight_dtype=wdt, **shape)
+    sizes = [_ws(d, T)[1] for T in range(0, 2100)] + [_ws(d, T)[1] for T in range(2100, 4200, 37)]
+    assert sizes == sorted(sizes)
+
+
 @pytest.mark.parametrize("field,value", [("top_k", 0), ("top_k", 9), ("router_mode", 3),
                                          ("weight_dtype", 7), ("param_dtype", 2),
                                          ("hidden", 0), ("n_experts", -1)])

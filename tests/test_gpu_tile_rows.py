@@ -6,7 +6,9 @@ import numpy as np
 import pytest
 
 from _cases import spec_for
+from moe_mi355x import _lib
 from moe_mi355x import synthetic as syn
+from moe_mi355x.device_layer import DeviceMoeLayer
 from moe_mi355x.quantize import quantize_moe_tensors
 from oracle import moe_oracle as orc
 from test_gpu_parity import LOWP_ABS, check_routing, run_device
@@ -38,3 +40,26 @@ def test_tile_rows(mi355x, stream, wdt, E, k, T, m_blk, frag):
     check_routing(views, ref, ref["logits"], t["mlp.gate.e_score_correction_bias"], spec,
                   f"{wdt} T={T}", x, t)
     assert float(np.max(np.abs(out - ref["out"]))) <= LOWP_ABS
+
+
+def test_reserved_once_serves_shorter_batches(mi355x, stream):
+    """513 tokens take one router slice less than 512: buffers reserved for 513 run 512."""
+    print("[gpu] reserve 513 tokens, run 512", flush=True)
+    shape = syn.MoeShape(syn.QWEN, 2048, 512, 2, 32, 32, 1.0, 1e-6, has_bias=False,
+                         has_shared_gate=True)
+    layer = DeviceMoeLayer.synthetic(mi355x, shape, 77, stream, weight_dtype="float16",
+                                     param_dtype="float32")
+    cfg = layer.config(top_k=2, router_mode=_lib.MX_ROUTER_SOFTMAX, routed_scaling=1.0, eps=1e-6)
+    x = syn.make_inputs(78, 513, shape.hidden)
+    try:
+        layer.prepare(cfg, 513)
+        got = layer.forward_numpy(cfg, x[:512])
+        fresh = DeviceMoeLayer.synthetic(mi355x, shape, 77, stream, weight_dtype="float16",
+                                         param_dtype="float32")
+        try:
+            want = fresh.forward_numpy(cfg, x[:512])
+        finally:
+            fresh.close()
+    finally:
+        layer.close()
+    assert np.array_equal(got, want)
