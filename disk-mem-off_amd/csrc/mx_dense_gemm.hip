@@ -63,6 +63,7 @@ struct GemmSeg {
   const void* scale;  // I8: fp16 scale of each weight row
   const float* res;  // residual added by the epilogue (same layout as y) or null
   float* y;       // [M, ldy] for slice 0; slice z at y + z * yslice
+  float* prod;    // I8: the product without the residual, same layout as y, or null
   int n;          // N of the segment
   int ldy;
   int nblk;       // column blocks of the segment
@@ -348,7 +349,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, OCC) void k_gemm_nt(
   // segment has one (read and written by the same lane, so it may alias the output).
   float* const ybase = sg.y + (size_t)blockIdx.y * p.yslice;
   const bool vec = (sg.ldy & 3) == 0 && ((uintptr_t)ybase & 15) == 0 &&
-                   ((uintptr_t)sg.res & 15) == 0;
+                   ((uintptr_t)sg.res & 15) == 0 && (!I8 || ((uintptr_t)sg.prod & 15) == 0);
   // Rows whose stride or base rules out 16-byte stores (the router logits, E + 1 columns):
   // the tile goes through LDS, then consecutive lanes store consecutive columns of a row,
   // in place of 4-byte stores spread over 16 rows per instruction.
@@ -370,6 +371,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, OCC) void k_gemm_nt(
         if (m < M && n < N) {
           const size_t o = (size_t)m * sg.ldy + n;
           ybase[o] = sg.res ? sg.res[o] + so[row * LDT + col] : so[row * LDT + col];
+          if (I8 && sg.prod) sg.prod[o] = so[row * LDT + col];
         }
       }
       return;
@@ -386,12 +388,16 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64, OCC) void k_gemm_nt(
       const int n = n0 + wn * WN + ni * 16 + 4 * q;
       if (vec && n + 3 < N) {
         float4_t v = acc[mi][ni];
+        if (I8 && sg.prod) *(float4_t*)(sg.prod + (size_t)m * sg.ldy + n) = v;
         if (rrow) v += *(const float4_t*)(rrow + n);
         *(float4_t*)(yrow + n) = v;
       } else {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          if (n + r < N) yrow[n + r] = rrow ? rrow[n + r] + acc[mi][ni][r] : acc[mi][ni][r];
+          if (n + r < N) {
+            yrow[n + r] = rrow ? rrow[n + r] + acc[mi][ni][r] : acc[mi][ni][r];
+            if (I8 && sg.prod) sg.prod[(size_t)m * sg.ldy + n + r] = acc[mi][ni][r];
+          }
       }
     }
   }
@@ -435,6 +441,7 @@ int prepare(GemmArgs& args, const void* a, int M, int K, int es, int wes, const 
     const MxGemmSeg& g = segs[i];
     if (!g.w || !g.y || g.n <= 0 || g.ldy < g.n) return MX_ERR_INVALID;
     if (g.res && kslice != K) return MX_ERR_INVALID;  // a residual needs the whole reduction
+    if (g.prod && (wes != 1 || !g.res)) return MX_ERR_INVALID;
     if (!mx_aligned16(g.w)) return MX_ERR_ALIGNMENT;
     if (wes == 1 && !g.scale) return MX_ERR_INVALID;
     if ((long)g.n * K * wes >= (1l << 31)) return MX_ERR_UNSUPPORTED;
@@ -442,6 +449,7 @@ int prepare(GemmArgs& args, const void* a, int M, int K, int es, int wes, const 
     args.seg[i].w_lo = g.w_lo;
     args.seg[i].scale = g.scale;
     args.seg[i].res = g.res;
+    args.seg[i].prod = g.prod;
     args.seg[i].y = g.y;
     args.seg[i].n = g.n;
     args.seg[i].ldy = g.ldy;
@@ -564,6 +572,7 @@ int mx_gemm(int wdt, const void* a, int M, int K, const MxGemmSeg* segs, int nse
         if (g.scale) t.scale = (const half_t*)g.scale + n0;
         t.y = g.y + n0;
         if (g.res) t.res = g.res + n0;
+        if (g.prod) t.prod = g.prod + n0;
         t.n = g.n - n0;
         tail[nt++] = t;
       }

@@ -53,8 +53,12 @@ __global__ __launch_bounds__(256) void k_residual(const float* x, float* y, long
 
 static_assert(MX_PROJ_MAX_SLICES <= MX_GEMM_MAX_SLICES, "k_residual adds either's slices");
 
-// Up to here the whole product is left in y (the header's view).
+// Up to here the product goes through y whatever its slices.
 #define MX_OUT_Y_TOKENS 64
+
+// Whether the whole product is left in y (the header's view): always for int8 weights, and
+// for fp16 ones up to MX_OUT_Y_TOKENS tokens.
+bool keep_product(int wdt, int T) { return wdt == MX_DT_I8 || T <= MX_OUT_Y_TOKENS; }
 
 // Reduction slices of an output projection.
 int out_slices(int wdt, int T, int N, int K) {
@@ -90,7 +94,7 @@ int mx_out_project(const MxDenseWork& dw, int ent, int wdt, const void* w, const
       return mx_gemm_slices(wdt, a, T, K, &g, slices, s);
     }
     if (!x || !out) return MX_ERR_INVALID;
-    const MxGemmSeg g{w, out, N, N, nullptr, x, scale};
+    const MxGemmSeg g{w, out, N, N, nullptr, x, scale, keep_product(wdt, T) ? y : nullptr};
     return mx_gemm(wdt, a, T, K, &g, 1, s);
   }
   return mx_project(dw, ent, wdt, T, N, K, a, y, s);
@@ -106,7 +110,7 @@ int mx_out_residual(int wdt, int T, int N, int K, float* y, const float* x, floa
   mx_clear_error();
   if (slices > 1)
     hipLaunchKernelGGL(k_residual<true>, grid, dim3(256), 0, s, x, y, n4, slices,
-                       T <= MX_OUT_Y_TOKENS, out);
+                       keep_product(wdt, T), out);
   else
     hipLaunchKernelGGL(k_residual<false>, grid, dim3(256), 0, s, x, y, n4, 1, false, out);
   return mx_launch_status();

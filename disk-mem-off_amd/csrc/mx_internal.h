@@ -143,6 +143,7 @@ struct MxGemmSeg {
   const void* w_lo = nullptr;  // mx_gemm_f16x2_slices: the low fp16 plane of w
   const float* res = nullptr;  // mx_gemm: y = res + a W^T (res [M, ldy], may alias y)
   const void* scale = nullptr;  // int8 W: fp16 scale of each row
+  float* prod = nullptr;        // int8 W with res: a W^T alone is stored here too
 };
 // fp16 a; W fp16 or per-row int8 (wdt), K a multiple of MX_GEMM_KMULT_F16 / MX_GEMM_KMULT_I8.
 int mx_gemm(int wdt, const void* a, int M, int K, const MxGemmSeg* segs, int nseg,
@@ -227,8 +228,9 @@ int mx_project(const MxDenseWork& w, int ent, int wdt, int T, int N, int K, cons
 // The projection that ends an attention block, out = x + a W^T (out may alias x), in two
 // stages: the product (into y, or straight into out where the GEMM's epilogue adds x), then
 // the residual sum (nothing to do in that case).  y holds mx_out_rows(T, N) rows of N floats:
-// the reduction slices of the product follow each other there, and the sum leaves the whole
-// product in the first T rows (up to 64 tokens; not written by the GEMM above).
+// the reduction slices of the product follow each other there.  The first T rows end up with
+// the whole product for int8 and fp32 weights at any length and for fp16 weights up to 64
+// tokens; above, the fp16 GEMM leaves them unwritten or holding a slice.
 size_t mx_out_rows(int T, int N);
 int mx_out_project(const MxDenseWork& dw, int ent, int wdt, const void* w, const void* scale,
                    int T, int N, int K, const void* a, float* y, const float* x, float* out,

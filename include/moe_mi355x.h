@@ -363,15 +363,19 @@ typedef struct MxLinearAttnViews {
   float* decay;  /* [T, n] exp(g)                                                       */
   float* o;      /* [T, n dv] recurrence output                                         */
   void* act;     /* [T, n dv] rms_norm(o) * silu(z), fp16 (fp32 for F32 weights)        */
-  float* y;      /* [T, H] act W_out^T; not written on the fused-GEMM path (below)      */
+  float* y;      /* [T, H] act W_out^T; unspecified for long fp16 inputs (below)        */
 } MxLinearAttnViews;
 
-/* Stages: rmsnorm, qkvz, ba, conv+gates, scan, gated norm, out, residual.  With fp16 or
- * int8 weights ba is computed in the qkvz launch (stage 2 is then empty, and the _profiled
- * events report ba's time under qkvz); short inputs form the conv and gates in the scan
- * launch (stage 3 is then empty).  With fp16 (int8) weights, T >= 65 and n dv a multiple of
- * 64 (128) the view y is not written: out = x + act W_out^T is formed in the out launch's
- * epilogue (stage 7 is then empty), or from the reduction slices of that launch.        */
+/* Stages: rmsnorm, qkvz, ba, conv+gates, scan, gated norm, out, residual.  Stages that
+ * another one's launch covers are empty, and the _profiled events report their time there:
+ *  - ba, in qkvz's launch, with fp16 or int8 weights up to 64 tokens and, above, where H is
+ *    a multiple of 64 (fp16) or 128 (int8);
+ *  - conv+gates, in scan's launch, up to 16 tokens with a conv kernel of 4 and key heads of
+ *    64, 128 or 256;
+ *  - residual, in out's launch, with fp16 (int8) weights, T >= 65 and n dv a multiple of
+ *    64 (128), unless the reduction is cut into slices.
+ * With fp16 weights, T >= 65 and n dv a multiple of 64 the contents of the view y are
+ * unspecified (the out launch may keep reduction slices there).                        */
 #define MX_LA_N_STAGES 8
 
 int mx_linear_attn_workspace_size(const MxLinearAttnDesc* desc, int32_t tokens,
@@ -433,15 +437,17 @@ typedef struct MxFullAttnViews {
   float* k;    /* [T, n_kv_heads head_dim] k, normalised and rotated in place           */
   float* v;    /* [T, n_kv_heads head_dim]                                              */
   void* act;   /* [T, n_heads head_dim] attn * sigmoid(gate), fp16 (fp32 for F32 weights) */
-  float* y;    /* [T, H] act W_o^T; not written on the fused-GEMM path (below)          */
+  float* y;    /* [T, H] act W_o^T; unspecified for long fp16 inputs (below)            */
 } MxFullAttnViews;
 
-/* Stages: rmsnorm, q, k, v, qk-norm+rope, attention, o, residual.  With fp16 or int8
- * weights k and v are computed in the q launch (stages 2 and 3 are then empty, and the
- * _profiled events report their time under q).  With fp16 (int8) weights, T >= 65 and
- * n_heads head_dim a multiple of 64 (128) the view y is not written: out = x + act W_o^T is
- * formed in the o launch's epilogue (stage 7 is then empty), or from the reduction slices of
- * that launch.                                                                          */
+/* Stages: rmsnorm, q, k, v, qk-norm+rope, attention, o, residual.  Stages that another
+ * one's launch covers are empty, and the _profiled events report their time there:
+ *  - k and v, in q's launch, with fp16 or int8 weights up to 64 tokens and, above, where H
+ *    is a multiple of 64 (fp16) or 128 (int8);
+ *  - residual, in o's launch, with fp16 (int8) weights, T >= 65 and n_heads head_dim a
+ *    multiple of 64 (128), unless the reduction is cut into slices.
+ * With fp16 weights, T >= 65 and n_heads head_dim a multiple of 64 the contents of the view
+ * y are unspecified (the o launch may keep reduction slices there).                    */
 #define MX_FA_N_STAGES 8
 
 int mx_full_attn_workspace_size(const MxFullAttnDesc* desc, int32_t tokens, size_t* nbytes);

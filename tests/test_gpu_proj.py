@@ -159,6 +159,43 @@ def test_linear_attention_gemm(mi355x, stream, wdt, hidden, heads, dk, dv, T):
     assert worst <= 1.0
 
 
+@pytest.mark.parametrize("kind,hidden,heads,dk,dv,T", [
+    ("linear", 384, 9, 32, 256, 65),    # 4 reduction slices
+    ("linear", 128, 4, 32, 1056, 129),  # 7 slices
+    ("linear", 256, 4, 32, 32, 130),    # one slice, 128 x 128 tiles
+    ("linear", 2048, 4, 32, 32, 2200),  # 128 x 256 tiles
+    ("linear", 2048, 4, 32, 32, 4500),  # whole rounds of 128 x 256 tiles, the rest on 128 x 128
+    ("full", 384, 4, 128, 128, 66),     # slices
+    ("full", 256, 4, 32, 32, 200),      # one slice
+])
+def test_int8_product_view_of_long_inputs(mi355x, stream, kind, hidden, heads, dk, dv, T):
+    """The view y holds the whole product act W^T for int8 weights at every length, however the
+    GEMM forms out = x + y."""
+    print(f"[gpu] int8 y view, {kind} hidden {hidden} K {heads * dv} T={T}", flush=True)
+    x = syn.make_inputs(31 + T, T, hidden)
+    if kind == "linear":
+        shape = syn.LinearAttnShape(hidden, heads, dk, dv, 4, 1e-6)
+        t = syn.make_linear_attn_tensors(shape, 30 + T, weight_dtype=np.float16, norm_noise=0.1)
+        w = _weights(t, (la.QKVZ, la.BA, la.OUT), "int8")[la.OUT]
+        layer = DeviceLinearAttnLayer.from_host(mi355x, t, stream)
+    else:
+        s = syn.FullAttnShape(hidden, heads, 2, dk, 0.25, 10000.0, 1e-6)
+        t = syn.make_full_attn_tensors(s, 30 + T, weight_dtype=np.float16, norm_noise=0.1)
+        w = _weights(t, (fa.Q, fa.K, fa.V, fa.O), "int8")[fa.O]
+        layer = DeviceFullAttnLayer.from_host(mi355x, t, heads, 2, dk, s.rotary_dim, s.rope_theta,
+                                              stream)
+    try:
+        out = layer.forward_numpy(x, 1e-6)
+        v = layer.runner.views(layer.desc(1e-6), T)
+        act = read_device(mi355x, v.act, np.float16, T * heads * dv, stream).reshape(T, -1)
+        y = read_device(mi355x, v.y, np.float32, T * hidden, stream).reshape(T, hidden)
+    finally:
+        layer.close()
+    _check("out", y.astype(np.float64), act.astype(np.float64), w)
+    # the sum with x, rounded once
+    assert np.all(np.abs(out - (x.astype(np.float64) + y)) <= 2.0 ** -23 * (np.abs(x) + np.abs(y)))
+
+
 def test_workspace_never_shrinks_with_tokens(mi355x):
     """A workspace sized for a batch serves every shorter one (the executors size it once)."""
     from moe_mi355x import _lib
