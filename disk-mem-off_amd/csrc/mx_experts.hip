@@ -824,6 +824,7 @@ static bool lds_eight_waves(int wdt, int K) {
 #ifndef MX_LDS_CHAIN8
 #define MX_LDS_CHAIN8 1  // slab chains for 8-wave blocks too
 #endif
+static_assert(MX_LDS_CHAIN >= 1, "slabs per block of the chained down launch");
 static int lds_slab_chain(bool gu, int wdt, int nw, const ExpertParams& p, int mt_max) {
   if (gu || wdt != MX_DT_F16 || MX_LDS_CHAIN < 2) return 1;
   if (nw != 4 && !(nw == 8 && MX_LDS_CHAIN8)) return 1;
@@ -1095,10 +1096,10 @@ static void launch_lds_tiled(int wdt, int nw, int ch, const ExpertParams& p, int
   if (wdt == MX_DT_F16) {
     kern = nw == 8 ? k_expert_lds<MX_DT_F16, GU, 8, 1, Y16, TILED>
                    : k_expert_lds<MX_DT_F16, GU, 4, 1, Y16, TILED>;
-    if constexpr (!GU)
-      if (ch == 2)
-        kern = nw == 8 && MX_LDS_CHAIN8 ? k_expert_lds<MX_DT_F16, false, 8, 2, Y16, TILED>
-                                        : k_expert_lds<MX_DT_F16, false, 4, 2, Y16, TILED>;
+    if constexpr (!GU && MX_LDS_CHAIN > 1)
+      if (ch > 1)
+        kern = nw == 8 ? k_expert_lds<MX_DT_F16, false, 8, MX_LDS_CHAIN, Y16, TILED>
+                       : k_expert_lds<MX_DT_F16, false, 4, MX_LDS_CHAIN, Y16, TILED>;
   }
   mx_clear_error();
   hipLaunchKernelGGL(kern, dim3(blocks), dim3(64 * nw), 0, s, p, mt_max, nblk);
