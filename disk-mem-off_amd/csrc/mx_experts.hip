@@ -929,26 +929,41 @@ __global__ __launch_bounds__((64 * NW), (LdsShape<WF>::OCC * 4 / NW)) void k_exp
 // Rows per m-tile.  A tile costs the direct-load kernel its height in activation fragment
 // loads whatever its group holds, and the 128-row kernel a barrier-paced walk; a tile too low
 // splits groups, and every tile of a group streams the group's weights (the later ones out of
-// L2).  The line is the average number of rows of a routed expert, pairs / n_experts
-// (`n_experts` 0: one group of all the rows), gate/up + down measured (MI355X, us):
+// L2).  The line is the average number of rows of a routed expert, pairs / n_experts; gate/up +
+// down measured (MI355X, us), even loads:
 //   int8: GLM-4.7 32 tokens (1.6 rows) 311 + 171 with 16 rows, 358 + 190 with 32; 64 tokens (3.2)
 //     381 + 214 with 16, 428 + 240 with 32, 610 + 313 with 64; 100 tokens (5) 420 + 251, 468 + 274,
 //     542 + 514 with 128; Qwen3-Next 400 tokens (7.8) 218 + 117, 207 + 130, 250 + 292; GLM-4.7 400
 //     tokens (20) 952 + 541, 724 + 365, 643 + 555; 1000 tokens (50) 1464 + 775 with 32, 787 + 672
 //     with 128.
 //   fp16: Qwen3-Next 24 tokens (0.5) 126 + 66 with 16, 131 + 67 with 32; 48 tokens (0.9) 206 + 109,
-//     209 + 111, 229 + 113 with 64; 100 tokens (2) 284 + 153, 280 + 154, 286 + 168 with 128; 200
-//     tokens (3.9) 327 + 179, 313 + 179, 308 + 187; GLM-4.7 64 tokens (3.2) 739 + 406, 736 + 399,
-//     822 + 442 with 64; 200 tokens (10) 801 + 491 with 32, 780 + 482 with 128.
-int mx_m_blk_for(int tokens, int weight_dtype, long pairs, int n_experts) {
-  if (tokens <= 16) return 16;
-  if (n_experts > 0 && weight_dtype == MX_DT_I8) {
-    if (pairs <= 8l * n_experts) return 16;
-    if (pairs <= 24l * n_experts) return 32;
-  } else if (n_experts > 0 && weight_dtype == MX_DT_F16) {
-    if (pairs <= n_experts) return 16;
-    if (pairs <= (tokens <= 64 ? 8l : 3l) * n_experts) return 32;
+//     209 + 111, 229 + 113 with 64; 100 tokens (2) 284 + 153, 280 + 154, 286 + 168 with 128; GLM-4.7
+//     64 tokens (3.2) 739 + 406, 736 + 399, 822 + 442 with 64; 200 tokens (10) 801 + 491 with 32,
+//     780 + 482 with 128.
+// Against 128 rows the int8 line stays at 14, where even loads still gain (20 rows: 10 %), for
+// the sake of uneven ones, whose largest groups split into many tiles (whole block, GLM-4.7 with a
+// correction bias of spread 0.04: 15 rows 966 us with 32-row tiles, 1019 with 128, 20 rows 1157 /
+// 1074, 24 rows 1317 / 1129; spread 0.08: 14 rows 883 / 884, 15 rows 945 / 891).  For fp16 it lies
+// at 2 rows, and at 3 where the shared expert, whose few 128-row tiles leave most CUs idle, is the
+// larger part of a token's work (whole block, hidden 2048, experts of 1024, 96 tokens: 64
+// experts, k = 2, 3 rows, shared 1024 179 / 170 and shared 4096 238 / 331; 32 experts, k = 1, 3 rows,
+// shared 1024 116 / 139); past 128 tokens its own tiles repeat its weights too often (128 experts,
+// k = 1, shared 1024: 160 tokens 224 / 216, 256 tokens 287 / 247).
+int mx_m_blk_for(const MxMoeDesc* d, int tokens) {
+  const long pairs = (long)tokens * d->top_k, E = d->n_experts;
+  if (tokens > 16 && d->weight_dtype == MX_DT_I8) {
+    if (pairs <= 8 * E) return 16;
+    if (pairs <= (tokens <= 64 ? 24 : 14) * E) return 32;
+  } else if (tokens > 16 && tokens <= 128 && d->weight_dtype == MX_DT_F16) {
+    const bool shared_heavy = d->shared_inter >= (long)d->top_k * d->inter;
+    if (pairs <= E) return 16;
+    if (pairs <= (tokens <= 64 ? 8 : shared_heavy ? 3 : 2) * E) return 32;
   }
+  return mx_m_blk_for(tokens, d->weight_dtype);
+}
+
+int mx_m_blk_for(int tokens, int weight_dtype) {
+  if (tokens <= 16) return 16;
   if (tokens <= 32) return 32;
   if (tokens <= 64 || weight_dtype == MX_DT_F32) return 64;
   return MX_PREFILL_M_BLK;

@@ -25,9 +25,10 @@ int mx_router_logits_split(const void* h16, const void* h16lo, const void* route
 // Upper bound of the m-tile list for `tokens` tokens at m_blk rows per tile.
 int mx_max_mtiles(int tokens, int top_k, int n_experts, int has_shared, int m_blk);
 
-// Rows per m-tile the expert kernels use for `tokens` tokens and `pairs` (token, slot) pairs
-// over n_experts routed experts (0: a single group of all the rows).
-int mx_m_blk_for(int tokens, int weight_dtype, long pairs = 0, int n_experts = 0);
+// Rows per m-tile the expert kernels use for `tokens` tokens of a block, and for a single
+// group of all the rows.
+int mx_m_blk_for(const MxMoeDesc* d, int tokens);
+int mx_m_blk_for(int tokens, int weight_dtype);
 
 // RMSNorm launch (vectorised when the row fits the register tile).
 // What the RMSNorm launch writes for the split-plane router GEMM: the router rows' fp16

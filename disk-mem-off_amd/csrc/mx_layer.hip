@@ -80,7 +80,7 @@ int layout(const MxMoeDesc* d, int T, void* ws, MxMoeViews* v, size_t* total,
   const int S = mx_router_splits_for(Tn, d->hidden, d->n_experts, d->has_shared_gate,
                                      d->param_dtype, d->weight_dtype);
   const bool split = mx_router_on_split(Tn, d->hidden, e1, d->weight_dtype);
-  const int m_blk = mx_m_blk_for(Tn, d->weight_dtype, (long)Tn * d->top_k, d->n_experts);
+  const int m_blk = mx_m_blk_for(d, Tn);
   const size_t P = (size_t)Tn * k;
   const size_t R = P + (has_sh ? Tn : 0);
   const size_t imax = d->inter > d->shared_inter ? d->inter : d->shared_inter;
@@ -140,7 +140,7 @@ int workspace_bound(const MxMoeDesc* d, int T, size_t* total) {
   auto key = [&](int t) {
     return Key{mx_router_splits_for(t, d->hidden, d->n_experts, d->has_shared_gate,
                                     d->param_dtype, d->weight_dtype),
-               mx_m_blk_for(t, d->weight_dtype, (long)t * d->top_k, d->n_experts),
+               mx_m_blk_for(d, t),
                mx_router_on_split(t, d->hidden, e1, d->weight_dtype)};
   };
   Key next = key(T > 0 ? T : 1);

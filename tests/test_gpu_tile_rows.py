@@ -1,7 +1,8 @@
 """Rows per m-tile chosen from the average rows of a routed expert: both sides of every line of
-the rule (int8: 8 and 24 rows; fp16: 1 row, 3 rows above 64 tokens, 8 rows up to 64), on both
-weight layouts.  The fp16 / int8 bar of the block's other parity tests: max abs 2e-2 against
-the fp32 evaluation with the same (dequantised) weights; routing tables bit for bit."""
+the rule (int8: 8 rows, 14 rows above 64 tokens, 24 up to 64; fp16 up to 128 tokens: 1 row, 2 rows
+above 64 tokens or 3 with a heavy shared expert, 8 rows up to 64), on both weight layouts.  The
+fp16 / int8 bar of the block's other parity tests: max abs 2e-2 against the fp32 evaluation with
+the same (dequantised) weights; routing tables bit for bit."""
 import numpy as np
 import pytest
 
@@ -17,15 +18,18 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("wdt,E,k,T,m_blk,frag", [
-    ("int8", 32, 4, 64, 16, True), ("int8", 32, 4, 65, 32, False), ("int8", 16, 4, 96, 32, True),
-    ("int8", 16, 4, 97, 128, True), ("int8", 64, 2, 257, 32, False), ("int8", 8, 2, 33, 32, True),
+    ("int8", 32, 4, 64, 16, True), ("int8", 32, 4, 65, 32, False), ("int8", 32, 4, 112, 32, True),
+    ("int8", 32, 4, 113, 128, True), ("int8", 8, 4, 48, 32, False), ("int8", 8, 4, 49, 64, True),
+    ("int8", 64, 2, 257, 32, False), ("int8", 8, 2, 33, 32, True),
     ("float16", 68, 2, 34, 16, True), ("float16", 64, 2, 33, 32, False),
     ("float16", 16, 2, 64, 32, True), ("float16", 16, 4, 34, 64, False),
-    ("float16", 64, 2, 96, 32, True), ("float16", 64, 2, 97, 128, True),
+    ("float16", 96, 2, 96, 32, True), ("float16", 96, 2, 97, 128, True),
+    ("float16", 32, 1, 96, 32, True), ("float16", 32, 1, 97, 128, False),  # heavy shared expert
+    ("float16", 200, 2, 128, 32, True), ("float16", 200, 2, 129, 128, True),
     ("float16", 200, 2, 100, 16, False)])
 def test_tile_rows(mi355x, stream, wdt, E, k, T, m_blk, frag):
     print(f"[gpu] tile rows {wdt} E={E} k={k} T={T} frag={frag}", flush=True)
-    shape = syn.MoeShape(syn.GLM, 128, E, k, 128, 64, 2.5, 1e-5)
+    shape = syn.MoeShape(syn.GLM, 128, E, k, 128, 128 if k == 1 else 64, 2.5, 1e-5)
     base = syn.make_tensors(shape, 300 + T, norm_noise=0.1)
     if wdt == "int8":
         t = quantize_moe_tensors(base)
