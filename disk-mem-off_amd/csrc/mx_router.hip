@@ -806,8 +806,10 @@ int mx_router_decode_launch(const MxMoeDesc* d, const MxMoeWeights* w, int T, co
   // Past one token per wave the one workgroup selects in rounds, four waves to a SIMD; a wave per
   // token over the chip and the dispatch in a launch of its own are shorter (us, one launch /
   // two): 512 experts 16 tokens 13.0 / 12.1, 24 tokens 16.9 / 12.1, 64 tokens 36.2 / 12.9; 160
-  // experts 16 tokens 9.7 / 10.5, 32 tokens 13.8 / 10.3, 64 tokens 22.0 / 10.6.
-  if (T > nw && d->top_k <= E) {
+  // experts 16 tokens 9.7 / 10.5, 32 tokens 13.8 / 10.3, 64 tokens 22.0 / 10.6.  With at most 64
+  // experts a round is short, and the second one costs less than the launch (block, 32 experts,
+  // 24 tokens 33.1 / 34.6, 32 tokens 35.4 / 36.1, 48 tokens 43.4 / 37.1).
+  if (T > (vpt == 1 ? 2 * nw : nw) && d->top_k <= E) {
     MX_TRY(mx_router_topk(logits, 1, b, d->param_dtype, T, E, d->top_k, d->router_mode,
                           d->norm_topk_prob, d->routed_scaling, d->has_shared_gate, ids, tw,
                           shared_w, s));
