@@ -804,6 +804,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(FA_H_WP
 #ifndef FA_D_PAIR
 #define FA_D_PAIR 1  // long and short query blocks paired on each CU
 #endif
+#define FA_D_RESIDENT 512  // blocks that run at once: two on each of 256 CUs
 
 // Max over the lanes l, l ^ 16, l ^ 32 and l ^ 48 (one query's four lane groups) without
 // going through LDS: permlane16_swap exchanges 16-lane rows 2k and 2k + 1 between its two
@@ -848,8 +849,12 @@ void k_fa_attn_d(const float* __restrict__ qg, const half_t* __restrict__ k16,
       // The XCD's first half of the blocks (the longest query blocks, longest first) takes
       // one slot of each CU and the second half the other: with the second half shortest
       // first, a CU's two query blocks have about the same sum of key tiles (the causal work
-      // of query block qx is proportional to nqb - qx).
-      if (FA_D_PAIR && (nqb & 1) == 0 && i >= per / 2) qx = nqb - 1 - (i - per / 2) / hpr;
+      // of query block qx is proportional to nqb - qx).  Only while all blocks are resident;
+      // with more, the short blocks would hold back the middling ones, so longest first
+      // (whole block, 16 heads: 2816 tokens, 704 blocks, 347 -> 331 us, 3584 tokens 430 -> 413,
+      // 6144 tokens, 768 blocks of two query sets, 810 -> 768).
+      if (FA_D_PAIR && nb <= FA_D_RESIDENT && (nqb & 1) == 0 && i >= per / 2)
+        qx = nqb - 1 - (i - per / 2) / hpr;
     }
   }
   const int q0 = (nqb - 1 - qx) * QB;
@@ -1125,7 +1130,7 @@ int launch_attn_h(const float* qg, const FaDims& m, int T, const FaPack& pk, voi
     // one set; 3000 tokens, 384 blocks, 140 against 116; 777 tokens 45 against 28; 24 tokens
     // 19 against 9.4).  8-wave blocks of one set: 84 us at 2000 tokens, 2-wave ones 101,
     // 4-wave ones 69 (two sets: 94).
-    if ((long)mx_ceil_div(T, 16 * FA_D_QS * FA_D_NW) * m.nh < 512) {
+    if ((long)mx_ceil_div(T, 16 * FA_D_QS * FA_D_NW) * m.nh < FA_D_RESIDENT) {
       const dim3 grid(mx_ceil_div(T, 16 * FA_D_NW), m.nh);
       hipLaunchKernelGGL((k_fa_attn_d<NC, FA_D_NW, 1>), grid, dim3(64 * FA_D_NW), 0, s, qg, k16,
                          v16t, m, T, Tp, sqrt_hd, (half_t*)act);

@@ -32,7 +32,10 @@ def stream(mi355x):
 @pytest.mark.parametrize("hd,nh,nkv,T", [
     (72, 4, 2, 33), (96, 4, 1, 70), (160, 4, 2, 40), (252, 2, 1, 129), (20, 4, 2, 65),
     (256, 8, 1, 1), (256, 8, 1, 16), (256, 8, 2, 17), (256, 8, 1, 32), (256, 8, 2, 64),
-    (256, 8, 2, 65), (256, 16, 2, 400), (128, 8, 2, 63), (128, 8, 1, 513), (256, 2, 2, 1030)])
+    (256, 8, 2, 65), (256, 16, 2, 400), (128, 8, 2, 63), (128, 8, 1, 513), (256, 2, 2, 1030),
+    # an even number of query blocks: all resident (512 blocks), and more than that with one and
+    # with two query sets per wave
+    (128, 16, 2, 2040), (128, 16, 2, 2170), (128, 32, 4, 2200)])
 def test_attention_matches_oracle(mi355x, stream, hd, nh, nkv, T):
     s = syn.FullAttnShape(128, nh, nkv, hd, 0.25 if hd % 8 == 0 else 0.5, 10000.0, 1e-6)
     if s.rotary_dim % 2:
