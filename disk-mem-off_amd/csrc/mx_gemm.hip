@@ -71,9 +71,10 @@ int out_slices(int wdt, int T, int N, int K) {
 
 size_t mx_out_rows(int T, int N) {
   // At least slices x T for every path's slice count, and never less for fewer tokens (a
-  // workspace sized for a batch serves the shorter ones): mx_proj splits T <= 64 rows of
-  // N < 8192 / slices columns, the GEMM as long as slices x its 128 x 128 tiles stay within
-  // MX_GEMM_SLICE_BLOCKS.
+  // workspace sized for a batch serves the shorter ones).  mx_proj doubles its slices while
+  // ceil(N / 16) times half of them is below 512, so N < 16384 / slices: with T <= 64 that is
+  // slices x T < 2^20 / N rows (and at most 256), inside `most`, about 2^22 / N.  The GEMM keeps
+  // slices times its 128 x 128 tiles within MX_GEMM_SLICE_BLOCKS.
   const size_t most = (size_t)128 * MX_GEMM_SLICE_BLOCKS / mx_ceil_div(N, 128);
   const size_t want = (size_t)MX_GEMM_MAX_SLICES * T;
   const size_t rows = want < most ? want : most;

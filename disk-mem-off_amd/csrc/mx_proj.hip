@@ -216,7 +216,8 @@ bool mx_proj_ok(int wdt, int T, int K) {
 }
 
 int mx_proj_slices(int wdt, int N, int K) {
-  // Two blocks per CU, while a wave keeps at least four chunks of its reduction.
+  // Up to 512 16-column units, while a wave keeps at least four chunks of its reduction: two
+  // blocks per CU up to 16 tokens, one of two units above.
   const int units = mx_ceil_div(N, 16), nch = mx_ceil_div(K, chunk_cols(wdt));
   int s = 1;
   while (s < MX_PROJ_MAX_SLICES && units * s < 512 && nch >= 4 * 4 * 2 * s) s *= 2;

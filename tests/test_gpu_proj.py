@@ -159,6 +159,34 @@ def test_linear_attention_gemm(mi355x, stream, wdt, hidden, heads, dk, dv, T):
     assert worst <= 1.0
 
 
+@pytest.mark.parametrize("T", [16, 17, 24, 32])
+def test_wide_fp16_products(mi355x, stream, T):
+    """qkvz and ba of 20,512 columns in all: on k_proj up to 16 tokens, on the GEMM from 17 (its
+    128-row tiles mostly padding), while the narrow out projection stays on k_proj."""
+    shape = syn.LinearAttnShape(128, 32, 128, 128, 4, 1e-6)
+    print(f"[gpu] wide fp16 projections T={T}", flush=True)
+    t = syn.make_linear_attn_tensors(shape, 60 + T, weight_dtype=np.float16, norm_noise=0.1)
+    w = _weights(t, (la.QKVZ, la.BA, la.OUT), "float16")
+    x = syn.make_inputs(61 + T, T, shape.hidden)
+    layer = DeviceLinearAttnLayer.from_host(mi355x, t, stream)
+    try:
+        out = layer.forward_numpy(x, shape.eps)
+        v = layer.runner.views(layer.desc(shape.eps), T)
+
+        def read(p, dt, n):
+            return read_device(mi355x, p, dt, T * n, stream).reshape(T, n).astype(np.float64)
+
+        h, act = read(v.h16, np.float16, 128), read(v.act, np.float16, 4096)
+        qkvz, ba = read(v.qkvz, np.float32, shape.qkvz_rows), read(v.ba, np.float32, shape.ba_rows)
+        y = read(v.y, np.float32, 128)
+    finally:
+        layer.close()
+    _check("qkvz", qkvz, h, w[la.QKVZ])
+    _check("ba", ba, h, w[la.BA])
+    _check("out", y, act, w[la.OUT])
+    assert np.array_equal(out, x + y.astype(np.float32))
+
+
 @pytest.mark.parametrize("kind,hidden,heads,dk,dv,T", [
     ("linear", 384, 9, 32, 256, 65),    # 4 reduction slices
     ("linear", 128, 4, 32, 1056, 129),  # 7 slices
