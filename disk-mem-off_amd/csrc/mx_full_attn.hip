@@ -1235,8 +1235,9 @@ int run_stage(int st, const MxFullAttnDesc* d, const MxFullAttnWeights* w, const
       if (!on_grouped(wdt, T, m.H, m.qw + 2 * m.kw)) return MX_OK;
       return mx_project(k.dw, 2, wdt, T, m.kw, m.H, h, k.v.v, s);
     case 4: {
-      // Long inputs: one block per token (777 tokens 11.9 us against 13.4 with 4 rows per
-      // block); short ones: 4 rows per block (200 tokens: 5.3 us against 6.6).
+      // Long inputs: one block per token; short ones: 4 rows per block.  By tokens alone; measured
+      // with 18 head rows of 256 (777 tokens 11.9 us against 13.4 with 4 rows per block, 200
+      // tokens 6.6 against 5.3).
       const int rows = m.nh + m.nkv, rpb = T >= 512 ? rows : 4;
       const dim3 grid(T + (f32 ? 0 : m.nkv * (pk.Tp / FA_KT)), mx_ceil_div(rows, rpb));
       mx_clear_error();

@@ -843,8 +843,9 @@ int run_stage(int st, const MxLinearAttnDesc* d, const MxLinearAttnWeights* w, c
     case 3: {
       if (short_ok(m, T)) return MX_OK;  // in stage 4
       // Tokens per thread: few enough that short inputs fill the chip, many enough that the
-      // K - 1 re-read inputs stay few (us with 4 / 8 / 16 tokens: 48 tokens 5.4 / 6.8 / 11.4; 100
-      // 6.4 / 8.4 / 12.4; 300 12.6 / 12.0 / 16.2; 1000 30.8 / 27.3 / 30.6; 2000 61.6 / 50.6 / 51.2).
+      // K - 1 re-read inputs stay few.  By tokens alone; measured with 12,320 channels and gates
+      // (us with 4 / 8 / 16 tokens: 48 tokens 5.4 / 6.8 / 11.4; 100 6.4 / 8.4 / 12.4; 300 12.6 /
+      // 12.0 / 16.2; 1000 30.8 / 27.3 / 30.6; 2000 61.6 / 50.6 / 51.2).
       const int tt = T <= 160 ? 4 : T <= 1536 ? 8 : 16;
       const dim3 grid(mx_ceil_div(m.C + m.n, 256), mx_ceil_div(T, tt));
       auto* kern = m.K == 4 ? (tt == 4 ? k_la_prep<4, 4> : tt == 8 ? k_la_prep<4, 8> : k_la_prep<4, 16>)
