@@ -940,10 +940,13 @@ __global__ __launch_bounds__((64 * NW), (LdsShape<WF>::OCC * 4 / NW)) void k_exp
 //     209 + 111, 229 + 113 with 64; 100 tokens (2) 284 + 153, 280 + 154, 286 + 168 with 128; GLM-4.7
 //     64 tokens (3.2) 739 + 406, 736 + 399, 822 + 442 with 64; 200 tokens (10) 801 + 491 with 32,
 //     780 + 482 with 128.
-// Against 128 rows the int8 line stays at 14, where even loads still gain (20 rows: 10 %), for
-// the sake of uneven ones, whose largest groups split into many tiles (whole block, GLM-4.7 with a
-// correction bias of spread 0.04: 15 rows 966 us with 32-row tiles, 1019 with 128, 20 rows 1157 /
-// 1074, 24 rows 1317 / 1129; spread 0.08: 14 rows 883 / 884, 15 rows 945 / 891).  For fp16 it lies
+// Against 128 rows the int8 line is set by uneven loads, whose largest groups split into many
+// tiles.  While an expert's gate/up weights fit an XCD's 4 MiB L2, the tiles after a group's first
+// cost little, and it lies at 24 rows (whole block with a correction bias of spread 0 / 0.04 / 0.08,
+// 512 experts of 512 on hidden 2048: 19 rows 481 / 524 / 498 us with 32-row tiles, 621 / 582 / 515
+// with 128, 23 rows 542 / 593 / 576 and 648 / 637 / 569); past that at 16 (GLM-4.7: 15 rows, spread
+// 0.04 966 / 1019, 20 rows 1157 / 1074, 24 rows 1317 / 1129; 0.08 14 rows 883 / 884, 15 rows 945 /
+// 891; experts of 1024 on hidden 4096: 15 rows, 0.04 435 / 514, 23 rows 551 / 535).  For fp16 it lies
 // at 2 rows, and at 3 where the shared expert, whose few 128-row tiles leave most CUs idle, is the
 // larger part of a token's work (whole block, hidden 2048, experts of 1024, 96 tokens: 64
 // experts, k = 2, 3 rows, shared 1024 179 / 170 and shared 4096 238 / 331; 32 experts, k = 1, 3 rows,
@@ -952,8 +955,9 @@ __global__ __launch_bounds__((64 * NW), (LdsShape<WF>::OCC * 4 / NW)) void k_exp
 int mx_m_blk_for(const MxMoeDesc* d, int tokens) {
   const long pairs = (long)tokens * d->top_k, E = d->n_experts;
   if (tokens > 16 && d->weight_dtype == MX_DT_I8) {
+    const bool in_l2 = 2l * d->hidden * d->inter <= (4l << 20);
     if (pairs <= 8 * E) return 16;
-    if (pairs <= (tokens <= 64 ? 24 : 14) * E) return 32;
+    if (pairs <= (tokens <= 64 || in_l2 ? 24 : 16) * E) return 32;
   } else if (tokens > 16 && tokens <= 128 && d->weight_dtype == MX_DT_F16) {
     const bool shared_heavy = d->shared_inter >= (long)d->top_k * d->inter;
     if (pairs <= E) return 16;

@@ -68,6 +68,32 @@ def test_moe_workspace_never_shrinks_with_tokens(wdt, shape):
     assert sizes == sorted(sizes)
 
 
+@pytest.mark.parametrize("wdt,hidden,inter,E,k,shared,T,m_blk", [
+    (_lib.MX_DT_I8, 5120, 1536, 160, 8, 1536, 160, 16),   # 8 rows per expert
+    (_lib.MX_DT_I8, 5120, 1536, 160, 8, 1536, 161, 32),
+    (_lib.MX_DT_I8, 5120, 1536, 160, 8, 1536, 320, 32),   # 16 rows, experts past 4 MiB
+    (_lib.MX_DT_I8, 5120, 1536, 160, 8, 1536, 321, 128),
+    (_lib.MX_DT_I8, 2048, 1024, 128, 8, 1024, 384, 32),   # 24 rows, experts of 4 MiB
+    (_lib.MX_DT_I8, 2048, 1024, 128, 8, 1024, 385, 128),
+    (_lib.MX_DT_I8, 2048, 1040, 128, 8, 1040, 257, 128),  # just past them
+    (_lib.MX_DT_I8, 5120, 1536, 16, 6, 1536, 64, 32),     # 24 rows up to 64 tokens
+    (_lib.MX_DT_I8, 5120, 1536, 15, 6, 1536, 64, 64),
+    (_lib.MX_DT_F16, 2048, 512, 512, 10, 512, 102, 32),   # 2 rows
+    (_lib.MX_DT_F16, 2048, 512, 512, 10, 512, 103, 128),
+    (_lib.MX_DT_F16, 2048, 512, 64, 2, 1024, 96, 32),     # 3 rows with a heavy shared expert
+    (_lib.MX_DT_F16, 2048, 512, 64, 2, 1023, 96, 128),
+    (_lib.MX_DT_F16, 2048, 512, 1024, 1, 512, 128, 16),
+    (_lib.MX_DT_F16, 2048, 512, 1024, 1, 512, 129, 128),
+    (_lib.MX_DT_F32, 2048, 512, 512, 10, 512, 65, 64)])
+def test_rows_per_tile(wdt, hidden, inter, E, k, shared, T, m_blk):
+    """Both sides of each line of the tile-height rule, read from the workspace views."""
+    d = _desc(weight_dtype=wdt, hidden=hidden, inter=inter, n_experts=E, top_k=k,
+              shared_inter=shared)
+    v = _lib.MxMoeViews()
+    rc = _lib.load().mx_moe_views(ctypes.byref(d), T, ctypes.c_void_p(1 << 12), ctypes.byref(v))
+    assert rc == _lib.MX_OK and v.m_blk == m_blk
+
+
 @pytest.mark.parametrize("field,value", [("top_k", 0), ("top_k", 9), ("router_mode", 3),
                                          ("weight_dtype", 7), ("param_dtype", 2),
                                          ("hidden", 0), ("n_experts", -1)])

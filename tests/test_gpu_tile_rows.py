@@ -1,5 +1,5 @@
 """Rows per m-tile chosen from the average rows of a routed expert: both sides of every line of
-the rule (int8: 8 rows, 14 rows above 64 tokens, 24 up to 64; fp16 up to 128 tokens: 1 row, 2 rows
+the rule (int8: 8 rows, and 24 for experts of this size; fp16 up to 128 tokens: 1 row, 2 rows
 above 64 tokens or 3 with a heavy shared expert, 8 rows up to 64), on both weight layouts.  The
 fp16 / int8 bar of the block's other parity tests: max abs 2e-2 against the fp32 evaluation with
 the same (dequantised) weights; routing tables bit for bit."""
@@ -18,8 +18,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("wdt,E,k,T,m_blk,frag", [
-    ("int8", 32, 4, 64, 16, True), ("int8", 32, 4, 65, 32, False), ("int8", 32, 4, 112, 32, True),
-    ("int8", 32, 4, 113, 128, True), ("int8", 8, 4, 48, 32, False), ("int8", 8, 4, 49, 64, True),
+    ("int8", 32, 4, 64, 16, True), ("int8", 32, 4, 65, 32, False), ("int8", 16, 4, 96, 32, True),
+    ("int8", 16, 4, 97, 128, True), ("int8", 8, 4, 48, 32, False), ("int8", 8, 4, 49, 64, True),
     ("int8", 64, 2, 257, 32, False), ("int8", 8, 2, 33, 32, True),
     ("float16", 68, 2, 34, 16, True), ("float16", 64, 2, 33, 32, False),
     ("float16", 16, 2, 64, 32, True), ("float16", 16, 4, 34, 64, False),
