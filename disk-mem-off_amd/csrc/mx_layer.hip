@@ -129,10 +129,25 @@ int layout(const MxMoeDesc* d, int T, void* ws, MxMoeViews* v, size_t* total,
 // fall as T grows: the router cuts its reduction into fewer slices once the rows fill the
 // chip (Qwen3-Next shape: 512 tokens take 5 MB more than 513), and higher m-tiles make
 // shorter lists.  Between two changes of those it only rises, so its value right before each
-// change and at T itself bound the rest.
+// change and at T itself bound the rest.  From WS_STEADY_TOKENS on the router has one slice
+// (two take at most half of a round's 1024 blocks, of at most 256 rows) and the tile rule its
+// highest tiles (at most 24 rows per expert for others, 1024 experts); all that changes there
+// is that the router's GEMMs end, at 2 GiB of activations.
+constexpr int WS_STEADY_TOKENS = 1 << 18;
+
 int workspace_bound(const MxMoeDesc* d, int T, size_t* total) {
   MX_TRY(layout(d, T, nullptr, nullptr, total));
   const int e1 = d->n_experts + (d->has_shared_gate ? 1 : 0);
+  auto raise_to = [&](int t) {
+    size_t n = 0;
+    MX_TRY(layout(d, t, nullptr, nullptr, &n));
+    if (n > *total) *total = n;
+    return MX_OK;
+  };
+  for (int esz : {2, 4}) {
+    const long t = ((1l << 31) - 1) / ((long)d->hidden * esz);
+    if (t > WS_STEADY_TOKENS && t < T) MX_TRY(raise_to((int)t));
+  }
   struct Key {
     int splits, m_blk;
     bool split_planes;
@@ -143,14 +158,12 @@ int workspace_bound(const MxMoeDesc* d, int T, size_t* total) {
                mx_m_blk_for(d, t),
                mx_router_on_split(t, d->hidden, e1, d->weight_dtype)};
   };
-  Key next = key(T > 0 ? T : 1);
-  for (int t = T - 1; t >= 1; --t) {
+  const int top = T < WS_STEADY_TOKENS ? T : WS_STEADY_TOKENS;
+  Key next = key(top > 0 ? top : 1);
+  for (int t = top - 1; t >= 1; --t) {
     const Key k = key(t);
-    if (k.splits != next.splits || k.m_blk != next.m_blk || k.split_planes != next.split_planes) {
-      size_t n = 0;
-      MX_TRY(layout(d, t, nullptr, nullptr, &n));
-      if (n > *total) *total = n;
-    }
+    if (k.splits != next.splits || k.m_blk != next.m_blk || k.split_planes != next.split_planes)
+      MX_TRY(raise_to(t));
     next = k;
   }
   return MX_OK;

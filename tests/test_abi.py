@@ -59,12 +59,16 @@ def test_workspace_size_grows_with_tokens():
     dict(hidden=5120, inter=1536, shared_inter=1536, n_experts=160, top_k=8),
     dict(hidden=2048, inter=512, shared_inter=512, n_experts=512, top_k=10, has_bias=0,
          has_shared_gate=1),
+    dict(hidden=512, inter=32, shared_inter=0, n_experts=8, top_k=1, param_dtype=_lib.MX_DT_F16),
     dict(hidden=64, inter=32, shared_inter=0, n_experts=1024, top_k=1)])
 def test_moe_workspace_never_shrinks_with_tokens(wdt, shape):
     """A workspace sized for a batch serves every shorter one (the runners size it once), although
     the router's slices and the m-tile lists get fewer as tokens grow."""
     d = _desc(weight_dtype=wdt, **shape)
-    sizes = [_ws(d, T)[1] for T in range(0, 2100)] + [_ws(d, T)[1] for T in range(2100, 4200, 37)]
+    edge = 2 ** 31 // (4 * d.hidden)  # the router's GEMMs end at 2 GiB of activations
+    tokens = [*range(0, 2100), *range(2100, 4200, 37), *range(4200, 300000, 20011),
+              131071, 131072, 131073, *sorted({edge - 1, edge, edge + 1, 2 * edge - 1, 2 * edge, 2 * edge + 1})]
+    sizes = [_ws(d, T)[1] for T in sorted(tokens)]
     assert sizes == sorted(sizes)
 
 
